@@ -297,9 +297,20 @@ __global__ __launch_bounds__(256) void k_pf_topk(PrefillArgs a) {
     else wave_topk<16>(a.logits + (uint64_t)t * a.E, a.E, a.k, a.ids + (uint64_t)t * a.k, a.w + (uint64_t)t * K1);
     float sw = 1.f;
     if (a.shared_gate_vec) {
+        // eight values per lane and load: 512 values of the row per wave instruction (value by value
+        // the dot was a chain of H / 64 load pairs: the kernel took 16.4 us with a gate vector, 7.3 without)
         float d = 0.f;
         const uint16_t *xp = a.x + (uint64_t)t * a.H;
-        for (int i = lane; i < a.H; i += 64) d = fmaf(bf2f(xp[i]), a.shared_gate_vec[i], d);
+        for (int i = 8 * lane; i < a.H; i += 512) {
+            const uint4 xw = ld16((const uint8_t *)(xp + i));   // (no alignment asked of either pointer)
+            const uint4 v0 = ld16((const uint8_t *)(a.shared_gate_vec + i)), v1 = ld16((const uint8_t *)(a.shared_gate_vec + i + 4));
+            const uint32_t xs[4] = {xw.x, xw.y, xw.z, xw.w}, vs[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                d = fmaf(bf2f(xs[q] & 0xFFFFu), __uint_as_float(vs[2 * q]), d);
+                d = fmaf(bf2f(xs[q] >> 16), __uint_as_float(vs[2 * q + 1]), d);
+            }
+        }
         d = wave_sum(d);
         sw = 1.0f / (1.0f + expf(-d));
     }

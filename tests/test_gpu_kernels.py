@@ -305,6 +305,29 @@ def test_moe_layer_norm_residual_gate(gpu):
     assert np.array_equal(got, (x + ffn).astype(np.float32))
 
 
+@pytest.mark.parametrize("E,H", [(1, 512), (15, 1024), (16, 512), (1023, 8192)])
+def test_route_gate_vector(gpu, E, H):
+    """The shared-expert gate as the router kernel's work-group of its own,
+    after an odd or even number of router rows (and a single one), at an
+    address of 4-byte alignment: the weight against fp64, the routing against
+    the same layer without a gate vector."""
+    from fomoe_amd import synthetic as S
+    say(f"route gate vector E={E} H={H}")
+    k = min(2, E)
+    shape = S.LayerShape(n_embd=H, inter=256, n_experts=E, k=k, shared=True)
+    L = S.build_layer(gpu, shape, 0, seed=81, zipf_s=1.1, norm=False)
+    h, gv = O.synth_f32(82, 0, 1.0, H), O.synth_f32(82, 1, 0.02, H)
+    dh, dout, dg = gpu.upload(h), gpu.alloc(4 * H), gpu.upload(np.concatenate([np.zeros(1, np.float32), gv]))
+    gpu.moe_layer(L.desc, dh, dout, 0)
+    ids0, w0, sw0 = gpu.last_routing(k)
+    L.desc.shared_gate_vec = dg.offset(4)
+    gpu.moe_layer(L.desc, dh, dout, 0)
+    ids, w, sw = gpu.last_routing(k)
+    assert sw0 == 1.0 and np.array_equal(ids, ids0) and np.array_equal(w, w0)
+    # fp32 sum of H products: within H/2 ulps of sum |h v| in the worst case, far less here; 1e-6 as above
+    assert abs(sw - 1 / (1 + np.exp(-float(h.astype(np.float64) @ gv)))) < 1e-6
+
+
 @pytest.mark.parametrize("E,k,shared", [(1024, 16, True), (1024, 16, False), (1024, 1, True), (17, 16, True)])
 def test_moe_layer_limits(gpu, E, k, shared):
     """The largest expert count and top-k the layer takes (E <= 1024,
