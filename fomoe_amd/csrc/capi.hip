@@ -726,8 +726,8 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
         HIPC(ensure(ctx->pf_ys, ctx->pf_ys_cap, sizeof(float) * (size_t)Tc * H));
     HIPC(ensure(ctx->pf_outp, ctx->pf_outp_cap, sizeof(float) * P * H));
     HIPC(ensure(ctx->pf_rsplit, ctx->pf_rsplit_cap, sizeof(uint16_t) * fo::prefill_router_ws_elems(E, Tc, H)));
-    // xsum [Tc x H/32] fp32, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
-    const size_t xs_bytes = sizeof(float) * (size_t)Tc * (H / 32), x16_bytes = 2 * (size_t)Tc * H;
+    // xsum [Tc x H/256 x 32] fp16, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
+    const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;
     HIPC(ensure(ctx->pf_xsum, ctx->pf_xsum_cap, xs_bytes + x16_bytes + sizeof(int32_t) * ((size_t)Tc + P)));
     fo::PrefillArgs a{};
     a.E = E; a.k = k; a.H = H; a.F = F;
@@ -745,7 +745,7 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
     a.pair_tok = ctx->pf_pairtok; a.tiles = ctx->pf_tiles; a.n_tiles = ctx->pf_ntiles;
     a.dtiles = ctx->pf_tiles + 4 * tcap;
     a.act_hi = ctx->pf_act; a.act_lo = ctx->pf_act + Pact; a.outp = ctx->pf_outp;
-    a.xsum = ctx->pf_xsum;
+    a.xsum = (uint16_t *)ctx->pf_xsum;
     a.x16 = (uint16_t *)((uint8_t *)ctx->pf_xsum + xs_bytes);
     a.xexp = (int32_t *)((uint8_t *)ctx->pf_xsum + xs_bytes + x16_bytes);
     a.pexp = a.xexp + Tc;

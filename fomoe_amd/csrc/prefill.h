@@ -48,8 +48,10 @@ struct PrefillArgs {
     int max_tiles;
     uint16_t *act_hi, *act_lo;   // [P x F] SwiGLU activation as bf16 hi + lo terms (a Q6_K
                                  // down projection rewrites act_hi as fp16 rows, scale in pexp)
-    float *xsum;                 // [T x H/32] sums of x over 32-value sub-blocks (Q4_K gate/up path)
-    uint16_t *x16;               // [T x H] fp16(x * 2^-xexp[t]) (Q4_K gate/up path)
+    uint16_t *xsum;              // [T x H/256 x 32] sums of x over 32-value sub-blocks as fp16 terms
+                                 // (pf_put_sum; Q4_K gate/up path)
+    uint16_t *x16;               // [T x H] fp16(x * 2^-xexp[t]), each eight values in the order of
+                                 // pf_x16_src (Q4_K gate/up path)
     int32_t *xexp;               // [T] per-token power-of-two scale of x16
     float *outp;                 // [P x H] fp32, per-pair down output
     int32_t *pexp;               // [P] power-of-two scale of the fp16 activation rows (Q6_K down)

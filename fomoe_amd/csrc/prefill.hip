@@ -844,10 +844,30 @@ __global__ __launch_bounds__(kPfGateWaves * 64, 4) void k_pf_gateup(PrefillArgs 
 constexpr int kWsWaves = 8;
 constexpr int kWsRows = 16 * kWsWaves;                // F rows per item
 
+// x16 keeps each eight values in the order q4_codes_f16 leaves a lane's eight
+// codes in: 0 2 1 3 4 6 5 7.
+FO_DEV int pf_x16_src(int i) { return ((i & 3) == 1 || (i & 3) == 2) ? i ^ 3 : i; }
+
+// Sub-block sum j of token t (already times 2^-s; |sum| < 2^20) / 32 as three
+// fp16 terms hi + mid + lo, within 2^-25 of it absolutely (the token's maximum
+// is 2^14 or more): the A operand of the min term's MFMA. Per (token,
+// super-block) 32 fp16: hi[8], mid[8], lo[8] over the sub-blocks, 8 zeros.
+FO_DEV void pf_put_sum(const PrefillArgs &a, int t, int j, float sum) {
+    uint16_t *p = a.xsum + ((uint64_t)t * (a.H / 256) + (j >> 3)) * 32 + (j & 7);
+    const float v = sum * 0.03125f;
+    const _Float16 hi = (_Float16)v;
+    const float r1 = v - (float)hi;
+    const _Float16 mid = (_Float16)r1, lo = (_Float16)(r1 - (float)mid);
+    p[0] = __builtin_bit_cast(uint16_t, hi);
+    p[8] = __builtin_bit_cast(uint16_t, mid);
+    p[16] = __builtin_bit_cast(uint16_t, lo);
+    p[24] = 0;
+}
+
 // Token prep for the fp16 path, one work-group per token: s = the power of
 // two that brings max|x| into [2^14, 2^15) (large and tiny rows alike),
 // x16 = fp16(x * 2^-s), the fp32 sums of the bf16 values over 32-value
-// sub-blocks (sequential) times 2^-s, and s.
+// sub-blocks (sequential) times 2^-s as fp16 terms, and s.
 __global__ __launch_bounds__(256) void k_pf_xprep(PrefillArgs a) {
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x, H = a.H;
@@ -862,14 +882,16 @@ __global__ __launch_bounds__(256) void k_pf_xprep(PrefillArgs a) {
     frexpf(m, &E);                                         // 2^(E-1) <= m < 2^E (m finite, nonzero)
     const int sx = E - 15;
     uint16_t *x16 = a.x16 + (uint64_t)t * H;
-    for (int i = tid; i < H; i += 256)
-        x16[i] = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(bf2f(xr[i]), -sx));
+    for (int i = tid; i < H; i += 256) {   // storage position i holds the value of pf_x16_src(i)
+        const int v = (i & ~7) | pf_x16_src(i & 7);
+        x16[i] = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(bf2f(xr[v]), -sx));
+    }
     const int nsb = H / 32;
     for (int j = tid; j < nsb; j += 256) {
         const uint16_t *p = xr + 32 * j;
         float sum = 0.f;
         for (int q = 0; q < 32; q++) sum = sum + bf2f(p[q]);
-        a.xsum[(uint64_t)t * nsb + j] = ldexpf(sum, -sx);
+        pf_put_sum(a, t, j, ldexpf(sum, -sx));
     }
     if (tid == 0) a.xexp[t] = sx;
 }
@@ -898,23 +920,23 @@ FO_DEV void pf_xprep_body(const PrefillArgs &a, uint32_t blk) {
     frexpf(m, &E);                                         // 2^(E-1) <= m < 2^E (m finite, nonzero)
     const int sx = E - 15;
     uint16_t *x16 = a.x16 + (uint64_t)t * H + (uint64_t)lane * V;
-    float *xs = a.xsum + (uint64_t)t * (H / 32) + lane * (V / 32);
     float sum = 0.f;
     for (int c = 0; c < nc; c++) {
         const uint4 w = *(const uint4 *)(xr + 8 * c);
         const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-        uint32_t o[4];
+        uint32_t hv[8];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const float f0 = bf2f(u[i] & 0xFFFFu), f1 = bf2f(u[i] >> 16);
             sum = sum + f0;
             sum = sum + f1;
-            o[i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(f0, -sx)) |
-                   ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(f1, -sx)) << 16);
+            hv[2 * i] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(f0, -sx));
+            hv[2 * i + 1] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)ldexpf(f1, -sx));
         }
-        *(uint4 *)(x16 + 8 * c) = make_uint4(o[0], o[1], o[2], o[3]);
+        *(uint4 *)(x16 + 8 * c) = make_uint4(hv[0] | (hv[2] << 16), hv[1] | (hv[3] << 16), hv[4] | (hv[6] << 16),
+                                             hv[5] | (hv[7] << 16));   // the order of pf_x16_src
         if ((c & 3) == 3) {
-            xs[c >> 2] = ldexpf(sum, -sx);
+            pf_put_sum(a, t, lane * (V / 32) + (c >> 2), ldexpf(sum, -sx));
             sum = 0.f;
         }
     }
@@ -931,42 +953,49 @@ __global__ __launch_bounds__(256) void k_pf_prep(PrefillArgs a, uint32_t n_rt) {
     else pf_xprep_body(a, blockIdx.x - n_rt);
 }
 
-// 6-bit (scale, min) of sub-block j from the 12 scale bytes (words y, z, w
-// of a Q4_K header; reference src/quant.c:72-80)
-FO_DEV void q4_scale_min(const uint4 &hdr, int j, uint32_t &sc, uint32_t &mn) {
-    const int jj = j & 3;
-    const uint32_t b0 = (hdr.y >> (8 * jj)) & 0xFFu, b4 = (hdr.z >> (8 * jj)) & 0xFFu, b8 = (hdr.w >> (8 * jj)) & 0xFFu;
-    const bool lo = j < 4;
-    sc = lo ? (b0 & 63) : ((b8 & 0xF) | ((b0 >> 2) & 0x30));
-    mn = lo ? (b4 & 63) : ((b8 >> 4) | ((b4 >> 2) & 0x30));
+// Scales of sub-blocks 2 kg and 2 kg + 1 of a Q4_K header (reference
+// src/quant.c:72-80, two at a time) as fp16 pairs for q4_codes_f16: scale *
+// 2^10 for the low nibbles (sub-block 2 kg), scale * 2^6 for the high ones.
+FO_DEV void q4_scale_pair(const uint4 &hdr, int kg, f16x2 (&sp)[2]) {
+    const int sh = 16 * (kg & 1);
+    const uint32_t A = hdr.w >> sh, B = hdr.y >> sh;
+    const uint32_t scp = kg < 2 ? (B & 0x3F3Fu) : ((A & 0x0F0Fu) | ((B >> 2) & 0x3030u));
+    const f16x2 m1024 = {(_Float16)-1024.f, (_Float16)-1024.f}, up = {(_Float16)1024.f, (_Float16)64.f};
+    // bytes under 0x64 are fp16 1024 + scale
+    const f16x2 s2 = (__builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, scp, 0x04010400u)) + m1024) * up;
+    sp[0] = (f16x2){s2[0], s2[0]};
+    sp[1] = (f16x2){s2[1], s2[1]};
 }
-
-// Eight codes of nibble h (0: low, 1: high) of q times the sub-block scale as
-// exact fp16. A byte b = code (h = 0) or 16 code (h = 1, the nibble masked in
-// place, no shift) becomes the fp16 1024 + b through byte permutes with 0x64;
-// with (sc, nsc) = q4_scale_f16(scale, h) one fma per pair gives code * scale:
-// (1024 + b) s - 1024 s with s = scale / 16^h, exact with one rounding
-// (|code * scale| <= 945).
-FO_DEV f16x8 q4_codes_f16(uint2 q, int h, f16x2 sc, f16x2 nsc) {
-    const uint32_t m = h ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-    const uint32_t w0 = q.x & m, w1 = q.y & m;
-    const uint32_t p[4] = {__builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u),
-                           __builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u),
-                           __builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u),
-                           __builtin_amdgcn_perm(0x64646464u, w1, 0x04030402u)};
+// The eight 6-bit mins of a Q4_K header as fp16 (sub-block order).
+FO_DEV f16x8 q4_mins_f16(const uint4 &hdr) {
+    const uint32_t lo = hdr.z & 0x3F3F3F3Fu, hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+    const f16x2 m1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
+    const uint32_t p[4] = {__builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u),
+                           __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u),
+                           __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u),
+                           __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)};
     u32x4 r;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        r[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, p[i]), sc, nsc));
+    for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p[i]) + m1024);
     return __builtin_bit_cast(f16x8, r);
 }
-// (scale / 16^h, -1024 scale / 16^h) as fp16 pairs, exact: the bits 0x6400 |
-// scale are 1024 + scale, 0x5400 | scale are 64 + scale / 16
-FO_DEV void q4_scale_f16(uint32_t scale, int h, f16x2 &sc, f16x2 &nsc) {
-    const f16x2 m1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
-    const f16x2 off = h ? (f16x2){(_Float16)-64.f, (_Float16)-64.f} : m1024;
-    sc = __builtin_bit_cast(f16x2, (scale * 0x10001u) | (h ? 0x54005400u : 0x64006400u)) + off;
-    nsc = sc * m1024;
+// Eight bytes of codes as two fp16 operands code * scale * 2^-14 (low
+// nibbles, high nibbles), exact. A nibble masked in place at bit 0 (bit 4) of
+// a half word is the fp16 subnormal code * 2^-24 (16 code * 2^-24); times
+// scale * 2^10 (scale * 2^6) it is the integer code * scale <= 945 times 2^-14,
+// a normal fp16 number. 18 instructions for 16 codes, where bytes put under
+// 0x64 by permutes and one fma per pair took 20. The values come out in the
+// order 0 2 1 3 4 6 5 7 (pf_x16_src).
+FO_DEV void q4_codes_f16(uint2 q, const f16x2 (&sp)[2], f16x8 &lo, f16x8 &hi) {
+    const uint32_t w[4] = {q.x, q.x >> 8, q.y, q.y >> 8};
+    u32x4 l, h;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, w[i] & 0x000F000Fu) * sp[0]);
+        h[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, w[i] & 0x00F000F0u) * sp[1]);
+    }
+    lo = __builtin_bit_cast(f16x8, l);
+    hi = __builtin_bit_cast(f16x8, h);
 }
 
 constexpr int kGbKC = 256;                            // K values per step
@@ -975,8 +1004,8 @@ constexpr uint32_t kGbW = 2 * kGbHalf;                // 4608 bytes: gate | up
 constexpr int kGbPieces = (kGbW + 1023) / 1024;       // 5 (the last one partial)
 constexpr uint32_t kGbArea = kGbPieces * 1024;        // a wave's LDS area (the partial piece lands whole)
 constexpr uint32_t kGbA = kPfMT * kGbKC * 2;          // 32 KiB token rows
-constexpr uint32_t kGbS = 8 * kPfMT * 4;              // 2 KiB sub-block sums
-constexpr uint32_t kGbLds = kGbA + kGbS + kWsWaves * kGbArea;   // 74 KiB
+constexpr uint32_t kGbS = kPfMT * 64;                 // 4 KiB sub-block sums (fp16 terms)
+constexpr uint32_t kGbLds = kGbA + kGbS + kWsWaves * kGbArea;   // 76 KiB
 
 __global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t gb_lds[];
@@ -984,9 +1013,13 @@ __global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs 
     __shared__ int s_exp[kPfMT];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, col = lane & 15, kg = lane >> 4;
     uint16_t *ab = (uint16_t *)gb_lds;
-    float *sb = (float *)(gb_lds + kGbA);
+    uint8_t *sb = gb_lds + kGbA;
     uint8_t *wb = gb_lds + kGbA + kGbS + w * kGbArea;    // [gate 16 x 144 | up 16 x 144]
-    const int H = a.H, nsb = H / 32, NQ = H / kGbKC, nfg = a.F / kWsRows;
+    const int H = a.H, NQ = H / kGbKC, nfg = a.F / kWsRows;
+    // the lane's token operand of MFMA pair c of token block 0 (see issue_x): + 256 bytes for the high nibbles
+    uint32_t aoff[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) aoff[c] = col * 512 + 16 * ((4 * c + kg) ^ col);
     const uint32_t rowb = (uint32_t)(H / 256) * 144;
     const int n_items = *a.n_tiles * nfg;
     for (;;) {
@@ -1018,14 +1051,18 @@ __global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs 
         };
         auto issue_x = [&](int q) {
             for (int q2 = w; q2 < 8 * nb; q2 += kWsWaves) {      // two token rows per wave instruction
-                const int m = 2 * q2 + (lane >> 5), c = (lane & 31) ^ (m & 15);
+                // 16-byte chunk 8 kg + 4 h + c of a row (lane group kg's values of MFMA (c, h)) lies at
+                // slot (4 (4 h + c) + kg) ^ (row & 15): the 16-lane groups of a 16-byte LDS read then
+                // touch 16 different bank groups
+                const int m = 2 * q2 + (lane >> 5), sl = (lane & 31) ^ (m & 15), c = ((sl & 3) << 3) | (sl >> 2);
                 const uint16_t *src = a.x16 + (uint64_t)__builtin_amdgcn_ds_bpermute(4 * m, tok) * H + q * kGbKC + 8 * c;
                 __builtin_amdgcn_global_load_lds((const void *)src,
                                                  (__attribute__((address_space(3))) void *)(ab + 2 * q2 * kGbKC), 16, 0, 0);
             }
-            if (w < 8)                                           // one sub-block's token sums per instruction
-                __builtin_amdgcn_global_load_lds((const void *)(a.xsum + (uint64_t)tok * nsb + q * 8 + w),
-                                                 (__attribute__((address_space(3))) void *)(sb + w * kPfMT), 4, 0, 0);
+            if (w < nb)                                          // the sums of token block w
+                __builtin_amdgcn_global_load_lds(
+                    (const void *)(a.xsum + ((uint64_t)__builtin_amdgcn_ds_bpermute(4 * (16 * w + (lane >> 2)), tok) * NQ + q) * 32 + 8 * (lane & 3)),
+                    (__attribute__((address_space(3))) void *)(sb + w * 1024), 16, 0, 0);
         };
         auto run = [&](auto NBC) {
             constexpr int NB = decltype(NBC)::value;
@@ -1040,53 +1077,64 @@ __global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs 
                 // Lane group kg owns sub-blocks 2 kg and 2 kg + 1 of the super-block
                 // (MFMA (c, h): lane group kg's 8 values are values 8c..8c+7 of
                 // sub-block 2 kg + h; the token operand is read in the same
-                // order), so each lane decodes two (scale, min) pairs instead of
-                // all eight.
-                auto pass = [&](const uint8_t *rw, f32x4 (&acc)[NB]) {
-                    const uint4 hw = *(const uint4 *)rw;
-                    f16x2 sp[2], nsp[2];
-                    float bm[2];                               // -dmin * m of sub-block 2 kg + h of row col
+                // order), so each lane decodes two scales instead of all eight.
+                // NM matrices together share every token operand read.
+                auto pass = [&](auto NMC, const uint8_t *rw, auto &...accs) {
+                    constexpr int NM = decltype(NMC)::value;
+                    f32x4 *acc[NM] = {&accs[0]...};
+                    f16x2 sp[NM][2];
+                    f32x4 dd[NM][NB];
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        uint32_t sc, mn;
-                        q4_scale_min(hw, 2 * kg + h, sc, mn);
-                        // sc as an fp16 pair: bits 0x6400 | sc = 1024 + sc, minus 1024
-                        q4_scale_f16(sc, h, sp[h], nsp[h]);
-                        bm[h] = -h2f(hw.x >> 16) * (float)mn;
+                    for (int g = 0; g < NM; g++) {
+                        q4_scale_pair(*(const uint4 *)(rw + g * kGbHalf), kg, sp[g]);
+#pragma unroll
+                        for (int tb = 0; tb < NB; tb++) dd[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
                     }
-                    f32x4 dd[NB];
-#pragma unroll
-                    for (int tb = 0; tb < NB; tb++) dd[tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
-                        const uint2 qw = *(const uint2 *)(rw + 16 + 32 * kg + 8 * c);   // sub-blocks 2 kg, 2 kg + 1
+                        f16x8 bw[NM][2];
 #pragma unroll
-                        for (int h = 0; h < 2; h++) {
-                            const f16x8 bw = q4_codes_f16(qw, h, sp[h], nsp[h]);
-                            const int chunk = 8 * kg + 4 * h + c;  // values 32 (2 kg + h) + 8 c
+                        for (int g = 0; g < NM; g++)   // 8 bytes of codes: sub-blocks 2 kg, 2 kg + 1
+                            q4_codes_f16(*(const uint2 *)(rw + g * kGbHalf + 16 + 32 * kg + 8 * c), sp[g], bw[g][0], bw[g][1]);
+#pragma unroll
+                        for (int h = 0; h < 2; h++)
 #pragma unroll
                             for (int tb = 0; tb < NB; tb++) {
-                                const int m = 16 * tb + col;
-                                const f16x8 av = *(const f16x8 *)(ab + m * kGbKC + 8 * (chunk ^ (m & 15)));
-                                dd[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw, dd[tb], 0, 0, 0);
+                                const f16x8 av = *(const f16x8 *)((const uint8_t *)ab + aoff[c] + 256 * h + 8192 * tb);
+#pragma unroll
+                                for (int g = 0; g < NM; g++)
+                                    dd[g][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw[g][h], dd[g][tb], 0, 0, 0);
                             }
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (NB > 2) __builtin_amdgcn_sched_barrier(0);
                     }
-                    const float d = h2f(hw.x);
+                    f16x8 mn[NM];
+                    float d[NM], dm[NM];
+#pragma unroll
+                    for (int g = 0; g < NM; g++) {
+                        const uint4 hw = *(const uint4 *)(rw + g * kGbHalf);
+                        mn[g] = q4_mins_f16(hw);
+                        d[g] = h2f(hw.x) * 16384.f;              // codes entered times 2^-14
+                        dm[g] = h2f(hw.x >> 16) * -32.f;         // sums entered divided by 32
+                    }
 #pragma unroll
                     for (int tb = 0; tb < NB; tb++) {
+                        // A: the sums of token 16 tb + col: hi, mid, lo terms of the eight sub-blocks, zeros
+                        const f16x8 sa = *(const f16x8 *)(sb + (16 * tb + col) * 64 + 16 * kg);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) acc[tb][i] = fmaf(d, dd[tb][i], acc[tb][i]);
+                        for (int g = 0; g < NM; g++) {
+                            const f32x4 ms = __builtin_amdgcn_mfma_f32_16x16x32_f16(sa, mn[g], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-                        for (int h = 0; h < 2; h++) {   // A: S of token 16 tb + col, sub-block 2 kg + h
-                            const float sa = sb[(2 * kg + h) * kPfMT + 16 * tb + col];
-                            acc[tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa, bm[h], acc[tb], 0, 0, 0);
+                            for (int i = 0; i < 4; i++)
+                                acc[g][tb][i] = fmaf(d[g], dd[g][tb][i], fmaf(dm[g], ms[i], acc[g][tb][i]));
                         }
                     }
                 };
-                pass(wb + col * 144, gA);
-                pass(wb + kGbHalf + col * 144, uA);
+                if constexpr (NB <= 2) {
+                    pass(std::integral_constant<int, 2>{}, wb + col * 144, gA, uA);
+                } else {
+                    pass(std::integral_constant<int, 1>{}, wb + col * 144, gA);
+                    pass(std::integral_constant<int, 1>{}, wb + kGbHalf + col * 144, uA);
+                }
                 __syncthreads();                               // the step's LDS is free for the next one
             }
             const int row = fg * kWsRows + 16 * w + col;
