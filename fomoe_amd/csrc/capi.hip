@@ -91,7 +91,7 @@ void gpu_free(gpu_ctx_t *c) {
                     c->act2, c->vec_in, c->vec_out, c->staging, c->pf_logits, c->pf_ids,
                     c->pf_w, c->pf_pairpos, c->pf_pairtok, c->pf_tiles, c->pf_ntiles,
                     c->pf_act, c->pf_outp, c->pf_xsum, c->pf_rsplit, c->sh_act, c->sh_ys,
-                    c->pf_ys};
+                    c->pf_ys, c->pf_segs};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     for (int b = 0; b < 2; b++) {
@@ -674,6 +674,52 @@ void gpu_synth_zipf_bias(uint64_t seed, uint64_t stream, int n, double s, float 
 
 
 // ------------------------------------------------------------------ prefill
+static size_t prefill_tile_cap(int Tc, int k, int E, bool sh) {
+    return (size_t)std::max(fo::prefill_max_tiles(Tc, k, E, sh), fo::prefill_max_tiles(Tc, 1, 1, false));
+}
+
+// Grow the workspace for passes of Tc tokens (T in all).
+static hipError_t size_prefill(gpu_ctx_t *ctx, int T, int Tc, int k, int E, int H, int F, int Fs, bool sh, bool own) {
+    const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
+    const size_t Pact = std::max(P * F, (size_t)Tc * Fs);   // activation elements of either pass
+    // xsum [Tc x H/256 x 32] fp16, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
+    const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;
+    hipError_t e = hipSuccess;
+    auto need = [&](auto *&p, size_t &cap, size_t bytes) { if (e == hipSuccess) e = ensure(p, cap, bytes); };
+    need(ctx->pf_logits, ctx->pf_logits_cap, sizeof(float) * (size_t)Tc * E);
+    need(ctx->pf_ids, ctx->pf_ids_cap, sizeof(int32_t) * (size_t)T * k);
+    need(ctx->pf_w, ctx->pf_w_cap, sizeof(float) * (size_t)T * (k + 1));
+    need(ctx->pf_pairpos, ctx->pf_pairpos_cap, sizeof(int32_t) * (size_t)Tc * (k + 1));
+    need(ctx->pf_pairtok, ctx->pf_pairtok_cap, sizeof(int32_t) * P);
+    need(ctx->pf_tiles, ctx->pf_tiles_cap, sizeof(int32_t) * 8 * prefill_tile_cap(Tc, k, E, sh));   // tiles, then double tiles
+    need(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256);
+    need(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + fo::kPfSeg - 1) / fo::kPfSeg) * E);
+    need(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact);
+    if (own)   // the shared pass's output [Tc x H] (its down rows, pairs in token order)
+        need(ctx->pf_ys, ctx->pf_ys_cap, sizeof(float) * (size_t)Tc * H);
+    need(ctx->pf_outp, ctx->pf_outp_cap, sizeof(float) * P * H);
+    need(ctx->pf_rsplit, ctx->pf_rsplit_cap, sizeof(uint16_t) * fo::prefill_router_ws_elems(E, Tc, H));
+    need(ctx->pf_xsum, ctx->pf_xsum_cap, xs_bytes + x16_bytes + sizeof(int32_t) * ((size_t)Tc + P));
+    return e;
+}
+
+// Give the prefill workspace back (nothing may be running on it).
+static void free_prefill(gpu_ctx_t *ctx) {
+    auto drop = [](auto *&p, size_t &cap) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    };
+    drop(ctx->pf_logits, ctx->pf_logits_cap);   drop(ctx->pf_ids, ctx->pf_ids_cap);
+    drop(ctx->pf_w, ctx->pf_w_cap);             drop(ctx->pf_pairpos, ctx->pf_pairpos_cap);
+    drop(ctx->pf_pairtok, ctx->pf_pairtok_cap); drop(ctx->pf_tiles, ctx->pf_tiles_cap);
+    drop(ctx->pf_ntiles, ctx->pf_ntiles_cap);   drop(ctx->pf_segs, ctx->pf_segs_cap);
+    drop(ctx->pf_act, ctx->pf_act_cap);         drop(ctx->pf_ys, ctx->pf_ys_cap);
+    drop(ctx->pf_outp, ctx->pf_outp_cap);       drop(ctx->pf_rsplit, ctx->pf_rsplit_cap);
+    drop(ctx->pf_xsum, ctx->pf_xsum_cap);
+    ctx->pf_T = 0;                              // the last prefill's routing is gone with it
+}
+
 int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_x, int n_tokens,
                     float *d_out, int flags) {
     if (!ctx) return -1;
@@ -702,33 +748,28 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
             return fail(ctx, -1, "moe prefill: Q4_K gate/up blobs must be 16-byte aligned "
                                  "(experts, shared, expert_stride, gate sizes)");
     }
-    // the grouping table holds n_experts x ceil(tokens/32) words: larger
-    // batches run as consecutive chunks (the results per token are the same)
-    const int Tc = std::min(T, (16384 / E) * 32);
     if (own && L->shared_gate_type == GGML_TYPE_Q4_K &&
         ((uintptr_t)L->shared % 16 || L->shared_gate_size % 16))
         return fail(ctx, -1, "moe prefill: a Q4_K shared blob and its gate size must be 16-byte aligned");
     const bool sh = L->shared != nullptr && !own;
     const int Fs = own ? L->shared_inter : F;
+    // Larger batches run as consecutive passes (the results per token are the
+    // same). A pass that the device has no memory for is halved, down to what
+    // one grouping table holds.
+    int Tc = fo::prefill_pass_tokens(T, k, E, sh);
+    const int t_least = std::min(T, fo::prefill_table_tokens(E));
+    for (;;) {
+        const hipError_t e = size_prefill(ctx, T, Tc, k, E, H, F, Fs, sh, own);
+        if (e == hipSuccess) break;
+        if (e != hipErrorOutOfMemory || Tc <= t_least) HIPC(e);
+        (void)hipGetLastError();
+        HIPC(hipStreamSynchronize(ctx->stream));
+        free_prefill(ctx);
+        Tc = std::max(t_least, Tc / 64 * 32);
+    }
     const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
-    const int max_tiles = fo::prefill_max_tiles(Tc, k, E, sh);
-    HIPC(ensure(ctx->pf_logits, ctx->pf_logits_cap, sizeof(float) * (size_t)Tc * E));
-    HIPC(ensure(ctx->pf_ids, ctx->pf_ids_cap, sizeof(int32_t) * (size_t)T * k));
-    HIPC(ensure(ctx->pf_w, ctx->pf_w_cap, sizeof(float) * (size_t)T * (k + 1)));
-    HIPC(ensure(ctx->pf_pairpos, ctx->pf_pairpos_cap, sizeof(int32_t) * (size_t)Tc * (k + 1)));
-    HIPC(ensure(ctx->pf_pairtok, ctx->pf_pairtok_cap, sizeof(int32_t) * P));
-    const size_t tcap = (size_t)std::max(max_tiles, fo::prefill_max_tiles(Tc, 1, 1, false));
-    HIPC(ensure(ctx->pf_tiles, ctx->pf_tiles_cap, sizeof(int32_t) * 8 * tcap));   // tiles, then double tiles
-    HIPC(ensure(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256));
-    const size_t Pact = std::max(P * F, (size_t)Tc * Fs);   // activation elements of either pass
-    HIPC(ensure(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact));
-    if (own)   // the shared pass's output [Tc x H] (its down rows, pairs in token order)
-        HIPC(ensure(ctx->pf_ys, ctx->pf_ys_cap, sizeof(float) * (size_t)Tc * H));
-    HIPC(ensure(ctx->pf_outp, ctx->pf_outp_cap, sizeof(float) * P * H));
-    HIPC(ensure(ctx->pf_rsplit, ctx->pf_rsplit_cap, sizeof(uint16_t) * fo::prefill_router_ws_elems(E, Tc, H)));
-    // xsum [Tc x H/256 x 32] fp16, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
+    const size_t tcap = prefill_tile_cap(Tc, k, E, sh), Pact = std::max(P * F, (size_t)Tc * Fs);
     const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;
-    HIPC(ensure(ctx->pf_xsum, ctx->pf_xsum_cap, xs_bytes + x16_bytes + sizeof(int32_t) * ((size_t)Tc + P)));
     fo::PrefillArgs a{};
     a.E = E; a.k = k; a.H = H; a.F = F;
     a.gate_type = L->gate_type; a.up_type = L->up_type; a.down_type = L->down_type;
@@ -750,6 +791,7 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
     a.xexp = (int32_t *)((uint8_t *)ctx->pf_xsum + xs_bytes + x16_bytes);
     a.pexp = a.xexp + Tc;
     a.rsplit = ctx->pf_rsplit;
+    a.segs = ctx->pf_segs;
     for (int t0 = 0; t0 < T; t0 += Tc) {
         const int n = std::min(Tc, T - t0);
         a.T = n;

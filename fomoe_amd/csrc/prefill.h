@@ -13,6 +13,9 @@
 namespace fo {
 
 constexpr int kPfMT = 64;        // tokens per GEMM tile (4 MFMA row blocks of 16)
+constexpr int kPfGroupLds = 16384;   // words of each grouping table (n_experts * ceil(tokens / 32))
+constexpr int kPfSeg = 512;          // tokens per grouping segment of a larger pass
+constexpr int kPfMaxPairs = 1 << 17; // pairs of a pass (its down outputs: 2 GiB at n_embd 4096)
 constexpr int kPfThin = 4;       // pairs of a thin tile (integer-MFMA Q6_K down path)
 constexpr int kPfGateWaves = 8;                   // gate/up work-group: 4 gate + 4 up waves (two per CU)
 constexpr int kPfGateRows = 32 * kPfGateWaves / 2; // F rows per gate/up work-group (32 per wave)
@@ -45,6 +48,8 @@ struct PrefillArgs {
     int32_t *n_tiles;            // [6]: tiles, tiles before the thin ones, work counter of the gate/up
                                  // kernel, double tiles, double tiles before those of thin experts,
                                  // the shared expert's first tile
+    int32_t *segs;               // [ceil(T / kPfSeg) x E] pairs per (segment, expert), then their first pair
+                                 // slots (passes above the grouping table's size)
     int max_tiles;
     uint16_t *act_hi, *act_lo;   // [P x F] SwiGLU activation as bf16 hi + lo terms (a Q6_K
                                  // down projection rewrites act_hi as fp16 rows, scale in pexp)
@@ -84,6 +89,15 @@ inline bool prefill_types_ok(int gate, int up, int down) {
 inline int prefill_pairs(int T, int k, bool shared) { return T * (k + (shared ? 1 : 0)); }
 inline int prefill_max_tiles(int T, int k, int E, bool shared) {
     return (prefill_pairs(T, k, shared) + kPfMT - 1) / kPfMT + E + (shared ? 1 : 0);
+}
+
+// Tokens of a pass: all that kPfMaxPairs pairs hold (weights are read once per
+// pass), and never fewer than one grouping table takes.
+inline int prefill_table_tokens(int E) { return (kPfGroupLds / E) * 32; }
+inline int prefill_pass_tokens(int T, int k, int E, bool shared) {
+    const int most = kPfMaxPairs / (k + (shared ? 1 : 0)) / 32 * 32, table = prefill_table_tokens(E);
+    const int n = most > table ? most : table;
+    return T < n ? T : n;
 }
 
 // Workspace of the bf16 router GEMM (rsplit, uint16 elements): the router's

@@ -319,9 +319,9 @@ __global__ __launch_bounds__(256) void k_pf_topk(PrefillArgs a) {
 
 // ============================================================ P3 grouping
 // LDS: per-expert token bitmap bm[e][W] and popcount prefixes pre[e][W],
-// W = ceil(T/32) words; counts and offsets over E+1 entries (entry E is the
-// shared expert, all T tokens).
-constexpr int kPfGroupLds = 16384;     // E*W words of each table
+// W = ceil(T/32) words (E * W <= kPfGroupLds, else segments of kPfSeg tokens);
+// counts and offsets over E+1 entries (entry E is the shared expert, all T
+// tokens).
 // Row stride of k_pf_group's tables: W rounded up to odd
 __host__ __device__ constexpr int pf_group_stride(int W) { return W | 1; }
 
@@ -361,23 +361,82 @@ FO_DEV void block_exclusive_scan64x4(uint64_t v0, uint64_t v1, uint64_t v2, uint
 // pairs < 2^21, full tiles < 2^16, per-expert-at-most-one classes < 2^12).
 FO_DEV uint32_t fld(uint64_t v, int lo, int bits) { return (uint32_t)((v >> lo) & ((1ull << bits) - 1)); }
 
-__global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a) {
+// Tokens [t0, t1) of the bitmaps: bit t - t0 of expert e's row for each routed
+// pair (t, e). Ends with a barrier.
+FO_DEV void pf_bitmaps(const PrefillArgs &a, uint32_t *bm, int Ws, int t0, int t1) {
+    const int tid = threadIdx.x, E = a.E, k = a.k;
+    for (int i = tid; i < E * Ws; i += 1024) bm[i] = 0;
+    __syncthreads();
+    for (int i = t0 * k + tid; i < t1 * k; i += 1024) {
+        const int t = i / k - t0, e = a.one_expert ? 0 : a.ids[i];
+        atomicOr(&bm[e * Ws + (t >> 5)], 1u << (t & 31));
+    }
+    __syncthreads();
+}
+
+// Popcount prefixes of expert tid's row; returns its bits.
+FO_DEV int pf_prefixes(const uint32_t *bm, uint32_t *pre, int Ws, int W) {
+    int cnt = 0;
+    for (int w = 0; w < W; w++) { pre[threadIdx.x * Ws + w] = cnt; cnt += __popc(bm[threadIdx.x * Ws + w]); }
+    return cnt;
+}
+
+// Pair slots of the routed pairs of tokens [t0, t1): s_off[e] is the slot of
+// expert e's first one among them.
+FO_DEV void pf_place(const PrefillArgs &a, const uint32_t *bm, const uint32_t *pre, const int *s_off, int Ws, int t0, int t1) {
+    const int k = a.k, K1 = k + 1;
+    for (int i = t0 * k + threadIdx.x; i < t1 * k; i += 1024) {
+        const int t = i / k, r = i - t * k, e = a.one_expert ? 0 : a.ids[i], tl = t - t0;
+        const uint32_t word = bm[e * Ws + (tl >> 5)];
+        const int pos = s_off[e] + (int)pre[e * Ws + (tl >> 5)] + __popc(word & ((1u << (tl & 31)) - 1u));
+        a.pair_tok[pos] = t;
+        a.pairpos[t * K1 + r] = pos;
+    }
+}
+
+// More tokens than one work-group's tables hold (E * ceil(T / 32) words) are
+// grouped in segments of kPfSeg tokens, a work-group each: k_pf_gcount counts
+// a segment's pairs per expert, k_pf_group turns the counts into the tile
+// tables and each (segment, expert)'s first pair slot, k_pf_gplace places the
+// segment's pairs.
+__global__ __launch_bounds__(1024) void k_pf_gcount(PrefillArgs a) {
+    __shared__ int s_cnt[1024];
+    const int t0 = blockIdx.x * kPfSeg, t1 = min(a.T, t0 + kPfSeg);
+    s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    for (int i = t0 * a.k + threadIdx.x; i < t1 * a.k; i += 1024) atomicAdd(&s_cnt[a.ids[i]], 1);
+    __syncthreads();
+    if ((int)threadIdx.x < a.E) a.segs[blockIdx.x * a.E + threadIdx.x] = s_cnt[threadIdx.x];
+}
+
+__global__ __launch_bounds__(1024) void k_pf_gplace(PrefillArgs a) {
+    extern __shared__ uint32_t lds[];
+    __shared__ int s_off[1024];
+    constexpr int W = kPfSeg / 32, Ws = pf_group_stride(W);
+    uint32_t *bm = lds, *pre = lds + a.E * Ws;
+    const int t0 = blockIdx.x * kPfSeg, t1 = min(a.T, t0 + kPfSeg);
+    if ((int)threadIdx.x < a.E) s_off[threadIdx.x] = a.segs[blockIdx.x * a.E + threadIdx.x];
+    pf_bitmaps(a, bm, Ws, t0, t1);
+    if ((int)threadIdx.x < a.E) pf_prefixes(bm, pre, Ws, W);
+    __syncthreads();
+    pf_place(a, bm, pre, s_off, Ws, t0, t1);
+}
+
+// n_seg: 0, or the segments k_pf_gcount counted (no bitmaps or placement here).
+__global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     extern __shared__ uint32_t lds[];
     const int tid = threadIdx.x;
     const int W = (a.T + 31) / 32, E = a.E, k = a.k, K1 = k + 1;
     const int Ws = pf_group_stride(W);   // odd: thread e's row walk below is free of bank conflicts
     uint32_t *bm = lds, *pre = lds + E * Ws;
-    for (int i = tid; i < E * Ws; i += 1024) bm[i] = 0;
-    __syncthreads();
-    for (int i = tid; i < a.T * k; i += 1024) {
-        const int t = i / k, e = a.one_expert ? 0 : a.ids[i];
-        atomicOr(&bm[e * Ws + (t >> 5)], 1u << (t & 31));
-    }
-    __syncthreads();
+    if (!n_seg) pf_bitmaps(a, bm, Ws, 0, a.T);
     const bool sh = a.shared != nullptr;
     int cnt = 0;
     if (tid < E) {
-        for (int w = 0; w < W; w++) { pre[tid * Ws + w] = cnt; cnt += __popc(bm[tid * Ws + w]); }
+        if (n_seg)
+            for (int q = 0; q < n_seg; q++) cnt += a.segs[q * E + tid];
+        else
+            cnt = pf_prefixes(bm, pre, Ws, W);
     } else if (tid == E && sh) {
         cnt = a.T;
     }
@@ -462,14 +521,14 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a) {
     // pair offsets of each expert for the placement pass
     __shared__ int s_off[1025];
     if (tid <= E) s_off[tid] = off;
+    if (n_seg && tid < E)
+        for (int q = 0, o = off; q < n_seg; q++) {
+            const int c = a.segs[q * E + tid];
+            a.segs[q * E + tid] = o;
+            o += c;
+        }
     __syncthreads();
-    for (int i = tid; i < a.T * k; i += 1024) {
-        const int t = i / k, r = i - t * k, e = a.one_expert ? 0 : a.ids[i];
-        const uint32_t word = bm[e * Ws + (t >> 5)];
-        const int pos = s_off[e] + (int)pre[e * Ws + (t >> 5)] + __popc(word & ((1u << (t & 31)) - 1u));
-        a.pair_tok[pos] = t;
-        a.pairpos[t * K1 + r] = pos;
-    }
+    if (!n_seg) pf_place(a, bm, pre, s_off, Ws, 0, a.T);
     if (sh)
         for (int t = tid; t < a.T; t += 1024) {
             const int pos = s_off[E] + t;
@@ -1746,7 +1805,7 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
     const bool okt = prefill_types_ok(a.gate_type, a.up_type, a.down_type);
     const int W = (a.T + 31) / 32;
     if (!okt || a.T <= 0 || a.E <= 0 || a.E > 1023 || a.k <= 0 || a.k > a.E || a.k > kMaxK ||
-        a.H <= 0 || a.H % 256 || a.H % (32 * kPfDownWaves) || a.H % (32 * kPfD16Waves) || a.F <= 0 || a.F % 256 || a.F % kPfGateRows || a.E * W > kPfGroupLds ||
+        a.H <= 0 || a.H % 256 || a.H % (32 * kPfDownWaves) || a.H % (32 * kPfD16Waves) || a.F <= 0 || a.F % 256 || a.F % kPfGateRows || (a.E * W > kPfGroupLds && (!a.segs || a.one_expert)) ||
         a.max_tiles < prefill_max_tiles(a.T, a.k, a.E, a.shared != nullptr))
         return hipErrorInvalidValue;
     const bool fp16_gateup = a.gate_type == GGML_TYPE_Q4_K && a.up_type == GGML_TYPE_Q4_K;
@@ -1780,9 +1839,19 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute((const void *)k_pf_group, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            2 * (kPfGroupLds + kMaxE) * (int)sizeof(uint32_t));
         if (e != hipSuccess) return e;
+        e = hipFuncSetAttribute((const void *)k_pf_gplace, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                2 * kMaxE * pf_group_stride(kPfSeg / 32) * (int)sizeof(uint32_t));
+        if (e != hipSuccess) return e;
         lds_attr = true;
     }
-    k_pf_group<<<1, 1024, 2 * (size_t)a.E * pf_group_stride(W) * sizeof(uint32_t), s>>>(a);
+    if (a.E * W <= kPfGroupLds) {
+        k_pf_group<<<1, 1024, 2 * (size_t)a.E * pf_group_stride(W) * sizeof(uint32_t), s>>>(a, 0);
+    } else {
+        const int n_seg = (a.T + kPfSeg - 1) / kPfSeg;
+        k_pf_gcount<<<n_seg, 1024, 0, s>>>(a);
+        k_pf_group<<<1, 1024, 0, s>>>(a, n_seg);
+        k_pf_gplace<<<n_seg, 1024, 2 * (size_t)a.E * pf_group_stride(kPfSeg / 32) * sizeof(uint32_t), s>>>(a);
+    }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (fp16_gateup) {   // exact fp16 operands

@@ -303,9 +303,9 @@ void gpu_gguf_free_moe_layer(gpu_ctx_t *ctx, gpu_moe_layer_t *L);
  * own), with gate/up types or an intermediate size of its own it runs first
  * as a one-expert pass whose output the routed pass adds at the shared weight;
  * n_experts <= 1023; with Q4_K gate/up, the experts and shared pointers,
- * expert_stride and the gate sizes must be multiples of 16 bytes (-1 else). A batch larger than the grouping table (n_experts *
- * ceil(n_tokens/32) > 16384) runs as consecutive chunks of
- * (16384 / n_experts) * 32 tokens with the same results per token. No
+ * expert_stride and the gate sizes must be multiples of 16 bytes (-1 else). A batch of more
+ * than 131072 (token, expert) pairs runs as consecutive passes, and so does one that
+ * the device has no workspace memory for, with the same results per token. No
  * counterpart in the reference, which decodes prompt tokens one at a time
  * (gpu_forward). */
 int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *layer, const uint16_t *d_x, int n_tokens,

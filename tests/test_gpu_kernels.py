@@ -1306,6 +1306,33 @@ def test_prefill_chunked_shared_own_types(gpu):
         assert e <= 3e-4
 
 
+@pytest.mark.parametrize("E,k,T,cut", [(512, 4, 1025, 1024), (512, 4, 1536, 512), (1023, 16, 513, 511),
+                                       (16, 4, 33000, 26208)])
+def test_prefill_pass_sizes(gpu, E, k, T, cut):
+    """Passes larger than one grouping table (E * ceil(T / 32) words: counted,
+    scanned and placed in 512-token segments, the last one of 1 token, a
+    whole one, 1 of 2) and a batch above a pass's pairs (131072 with the
+    shared expert's): bit-identical to two separate calls, whose first part
+    fits one table or pass (F = 256: every expert on the same GEMM path), with
+    the same routing."""
+    from fomoe_amd import synthetic as S
+    say(f"prefill passes E={E} k={k} T={T}")
+    shape = S.LayerShape(n_embd=256, inter=256, n_experts=E, k=k, shared=True)
+    H = shape.n_embd
+    L = S.build_layer(gpu, shape, 0, seed=91, zipf_s=1.1, norm=False)
+    dx, dout, d2 = S.tokens_bf16(gpu, T, H, seed=92), gpu.alloc(4 * T * H), gpu.alloc(4 * T * H)
+    gpu.moe_prefill(L.desc, dx, T, dout, FA.MOE_RESIDUAL)
+    got = gpu.download(dout, np.uint32, T * H)
+    ids, w = gpu.prefill_routing(T, k)
+    parts = []
+    for t0, n in ((0, cut), (cut, T - cut)):
+        gpu.moe_prefill(L.desc, dx.offset(2 * t0 * H), n, d2.offset(4 * t0 * H), FA.MOE_RESIDUAL)
+        parts.append(gpu.prefill_routing(n, k))
+    assert np.array_equal(ids, np.concatenate([p[0] for p in parts]))
+    assert np.array_equal(w, np.concatenate([p[1] for p in parts]))
+    assert np.array_equal(got, gpu.download(d2, np.uint32, T * H))
+
+
 @pytest.mark.parametrize("down", [O.Q6_K, O.Q5_K])
 def test_prefill_repeatable(gpu, down):
     """Work-groups take their items from atomic counters, so which work-group
