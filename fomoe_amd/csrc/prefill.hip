@@ -891,17 +891,28 @@ __global__ __launch_bounds__(kPfGateWaves * 64, 4) void k_pf_gateup(PrefillArgs 
 // fp16 rows are exact for every value above 2^-28 of the row maximum and off
 // by at most 2^-39 of it below), which the epilogue undoes.
 //
-// Work item = (tile, 128 rows of F); work-group = 8 waves, wave w owns the
-// 16 gate and 16 up rows 16w..16w+15 of the item. K runs in steps of one
-// super-block: per step each wave's rows (2 x 16 x 144 bytes) go from HBM
-// straight into its own LDS area by direct global->LDS loads (1 KiB
-// coalesced pieces, no registers), and the work-group shares the step's token
-// rows (<= 64 x 256 fp16, swizzled) and sub-block sums, staged the same way.
-// 74 KiB of LDS and <= 128 VGPRs: two work-groups share a CU, and the loads
-// of one overlap the arithmetic of the other. Work-groups take items from a
-// counter (reset by k_pf_group).
-constexpr int kWsWaves = 8;
-constexpr int kWsRows = 16 * kWsWaves;                // F rows per item
+// Work item = (tile, 128 rows of F); work-group = 4 waves, wave w owns 32 gate
+// rows and the same 32 up rows of the item, as four blocks of 16 that share
+// every token operand read (one LDS read feeds four MFMAs; with 16 + 16 rows in
+// each of eight waves it fed two or, above 32 tokens, one, and the LDS reads
+// took longer than the MFMAs). K runs in steps of one super-block: per step each
+// wave's rows (64 x 144 bytes) go from HBM straight into its own LDS area by
+// direct global->LDS loads (1 KiB coalesced pieces, no registers), and the
+// work-group shares the step's token rows (<= 64 x 256 fp16, swizzled) and
+// sub-block sums, staged the same way. 72 KiB of LDS and <= 256 VGPRs: two
+// work-groups share a CU, and the loads of one overlap the arithmetic of the
+// other. Work-groups take their first item by index and the others from a counter
+// (reset by k_pf_group). What bounds it: the steps' latencies at two waves per
+// SIMD, not a unit (at 512 tokens VALU ~40 %, MFMA ~22 %, LDS ~15 % busy) and,
+// for tiles of few tokens, HBM (1.1 x the distinct bytes fetched). Trace, against
+// eight waves of 16 + 16 rows: 16 / 512 / 4096 tokens 66 / 331 / 1303 us
+// against 73 / 338 / 1360. Measured slower: one work-group per CU with both
+// operands double-buffered by direct loads (218 / 1466 us at 512 / 4096 tokens
+// for the tiles above 16 tokens, which take 177 / 1025 us this way), or with
+// eight waves and the weights a step ahead in registers (221 / 1242); eight
+// waves of 16 + 16 rows at 128 VGPRs sharing each read between gate and up (176 / 1115);
+// tiles of at most 16 tokens as a kernel of their own that streams 576-byte (or
+// 288-byte) row pieces ahead through registers: 173 + 177 us at 512 tokens.
 
 // x16 keeps each eight values in the order q4_codes_f16 leaves a lane's eight
 // codes in: 0 2 1 3 4 6 5 7.
@@ -1018,7 +1029,8 @@ __global__ __launch_bounds__(256) void k_pf_prep(PrefillArgs a, uint32_t n_rt) {
 FO_DEV void q4_scale_pair(const uint4 &hdr, int kg, f16x2 (&sp)[2]) {
     const int sh = 16 * (kg & 1);
     const uint32_t A = hdr.w >> sh, B = hdr.y >> sh;
-    const uint32_t scp = kg < 2 ? (B & 0x3F3Fu) : ((A & 0x0F0Fu) | ((B >> 2) & 0x3030u));
+    const uint32_t lom = (uint32_t)((kg >> 1) - 1);   // all ones for sub-blocks 0..3 (a select, no branch)
+    const uint32_t scp = (B & 0x3F3Fu & lom) | (((A & 0x0F0Fu) | ((B >> 2) & 0x3030u)) & ~lom);
     const f16x2 m1024 = {(_Float16)-1024.f, (_Float16)-1024.f}, up = {(_Float16)1024.f, (_Float16)64.f};
     // bytes under 0x64 are fp16 1024 + scale
     const f16x2 s2 = (__builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, scp, 0x04010400u)) + m1024) * up;
@@ -1057,163 +1069,168 @@ FO_DEV void q4_codes_f16(uint2 q, const f16x2 (&sp)[2], f16x8 &lo, f16x8 &hi) {
     hi = __builtin_bit_cast(f16x8, h);
 }
 
-constexpr int kGbKC = 256;                            // K values per step
-constexpr uint32_t kGbHalf = 16 * 144;                // a wave's 16 rows of one matrix per step
-constexpr uint32_t kGbW = 2 * kGbHalf;                // 4608 bytes: gate | up
-constexpr int kGbPieces = (kGbW + 1023) / 1024;       // 5 (the last one partial)
-constexpr uint32_t kGbArea = kGbPieces * 1024;        // a wave's LDS area (the partial piece lands whole)
-constexpr uint32_t kGbA = kPfMT * kGbKC * 2;          // 32 KiB token rows
-constexpr uint32_t kGbS = kPfMT * 64;                 // 4 KiB sub-block sums (fp16 terms)
-constexpr uint32_t kGbLds = kGbA + kGbS + kWsWaves * kGbArea;   // 76 KiB
+constexpr uint32_t kGuHalf = 16 * 144;                // 16 rows of one matrix, one super-block
+constexpr uint32_t kGuA = kPfMT * 512;                // 32 KiB of token rows
+constexpr uint32_t kGuS = kPfMT * 64;                 // 4 KiB: their sub-block sums (fp16 terms)
+constexpr uint32_t kGuW = 4 * kGuHalf;                // a wave's weights: 32 gate and 32 up rows
+constexpr int kGuWaves = 4;
+constexpr uint32_t kGuLds = kGuA + kGuS + kGuWaves * kGuW;   // 72 KiB: two work-groups per CU
 
-__global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t gb_lds[];
-    __shared__ int s_item;
-    __shared__ int s_exp[kPfMT];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, col = lane & 15, kg = lane >> 4;
-    uint16_t *ab = (uint16_t *)gb_lds;
-    uint8_t *sb = gb_lds + kGbA;
-    uint8_t *wb = gb_lds + kGbA + kGbS + w * kGbArea;    // [gate 16 x 144 | up 16 x 144]
-    const int H = a.H, NQ = H / kGbKC, nfg = a.F / kWsRows;
-    // the lane's token operand of MFMA pair c of token block 0 (see issue_x): + 256 bytes for the high nibbles
-    uint32_t aoff[4];
+// One super-block of NM blocks of 16 weight rows (row col of block g at rw +
+// g * gstride, 144 bytes of it) times NB blocks of 16 tokens: token operand
+// (c, h) of block tb at ab + aoff[c] + 256 h + 8192 tb, its sums at sb + 1024
+// tb. Lane group kg owns sub-blocks 2 kg and 2 kg + 1 (MFMA (c, h): its eight
+// values are values 8c..8c+7 of sub-block 2 kg + h in pf_x16_src order), so a
+// lane decodes two scales instead of eight; the NM blocks share every token
+// operand read. Each (row, token) sees the same operations in the same order
+// whatever NM and NB.
+template <int NM, int NB>
+FO_DEV void q4_super_block(f32x4 (&acc)[NM][NB], const uint8_t *rw, uint32_t gstride, const uint8_t *ab,
+                           const uint32_t (&aoff)[4], const uint8_t *sb, int col, int kg) {
+    f16x2 sp[NM][2];
+    f32x4 dd[NM][NB];
+#pragma unroll
+    for (int g = 0; g < NM; g++) {
+        q4_scale_pair(*(const uint4 *)(rw + g * gstride), kg, sp[g]);
+#pragma unroll
+        for (int tb = 0; tb < NB; tb++) dd[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        f16x8 bw[NM][2];
+#pragma unroll
+        for (int g = 0; g < NM; g++)
+            q4_codes_f16(*(const uint2 *)(rw + g * gstride + 16 + 32 * kg + 8 * c), sp[g], bw[g][0], bw[g][1]);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int tb = 0; tb < NB; tb++) {
+                const f16x8 av = *(const f16x8 *)(ab + aoff[c] + 256 * h + 8192 * tb);
+#pragma unroll
+                for (int g = 0; g < NM; g++)
+                    dd[g][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw[g][h], dd[g][tb], 0, 0, 0);
+            }
+        if constexpr (NM * NB > 8) __builtin_amdgcn_sched_barrier(0);   // keeps the live operands few
+    }
+    f16x8 mn[NM];
+    float d[NM], dm[NM];
+#pragma unroll
+    for (int g = 0; g < NM; g++) {
+        const uint4 hw = *(const uint4 *)(rw + g * gstride);
+        mn[g] = q4_mins_f16(hw);
+        d[g] = h2f(hw.x) * 16384.f;              // codes entered times 2^-14
+        dm[g] = h2f(hw.x >> 16) * -32.f;         // sums entered divided by 32
+    }
+#pragma unroll
+    for (int tb = 0; tb < NB; tb++) {
+        // A: the sums of token 16 tb + col: hi, mid, lo terms of the eight sub-blocks, zeros
+        const f16x8 sa = *(const f16x8 *)(sb + (16 * tb + col) * 64 + 16 * kg);
+#pragma unroll
+        for (int g = 0; g < NM; g++) {
+            const f32x4 ms = __builtin_amdgcn_mfma_f32_16x16x32_f16(sa, mn[g], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[g][tb][i] = fmaf(d[g], dd[g][tb][i], fmaf(dm[g], ms[i], acc[g][tb][i]));
+        }
+    }
+}
+
+// Rows [row, row + 16) of F for token block tb: act = silu(gate) * up as bf16 hi + lo.
+FO_DEV void q4_finish(const PrefillArgs &a, const int *s_exp, int p0, int n, int row, const f32x4 &g4, const f32x4 &u4,
+                      int tb, int col, int kg) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int m = 16 * tb + 4 * kg + i;
+        if (m < n) {
+            const int sx = s_exp[m];
+            const float g = ldexpf(g4[i], sx), u = ldexpf(u4[i], sx);
+            const float val = (g / (1.0f + expf(-g))) * u;
+            const __bf16 hi = (__bf16)val;
+            const __bf16 lo = (__bf16)(val - (float)hi);
+            const uint64_t o = (uint64_t)(p0 + m) * a.F + row + col;
+            a.act_hi[o] = __builtin_bit_cast(uint16_t, hi);
+            a.act_lo[o] = __builtin_bit_cast(uint16_t, lo);
+        }
+    }
+}
+
+// The lane's token operand of MFMA pair c of token block 0: chunk 8 kg + 4 h +
+// c of a row (16 bytes) lies at slot (4 (4 h + c) + kg) ^ (row & 15), so that
+// the 16-lane groups of a 16-byte LDS read touch 16 different bank groups.
+FO_DEV void q4_token_offsets(uint32_t (&aoff)[4], int col, int kg) {
 #pragma unroll
     for (int c = 0; c < 4; c++) aoff[c] = col * 512 + 16 * ((4 * c + kg) ^ col);
-    const uint32_t rowb = (uint32_t)(H / 256) * 144;
+}
+// The chunk at slot (lane & 31) of row m.
+FO_DEV int q4_token_chunk(int lane, int m) {
+    const int sl = (lane & 31) ^ (m & 15);
+    return ((sl & 3) << 3) | (sl >> 2);
+}
+
+__global__ __launch_bounds__(64 * kGuWaves, 2) void k_pf_gateup_f16(PrefillArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t gu_lds[];
+    __shared__ int s_item;
+    __shared__ int s_exp[kPfMT];
+    constexpr int NW = kGuWaves;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, kg = lane >> 4;
+    uint8_t *const wb = gu_lds + kGuA + kGuS + w * kGuW;    // [gate 32 rows | up 32 rows] x 144 bytes
+    const uint8_t *const sb = gu_lds + kGuA;
+    const int H = a.H, NQ = H / 256, nfg = a.F / (32 * NW);
+    const uint32_t rowb = (uint32_t)NQ * 144;
+    uint32_t aoff[4];
+    q4_token_offsets(aoff, col, kg);
     const int n_items = *a.n_tiles * nfg;
-    for (;;) {
-        if (tid == 0) s_item = atomicAdd(a.n_tiles + 2, 1);
-        __syncthreads();
-        const int item = s_item;
-        if (item >= n_items) break;
+    for (int item = blockIdx.x; item < n_items;) {
         const int ti = item / nfg, fg = item - ti * nfg;
-        const int tile = a.tiles[4 * ti + 3];                    // tiles in decreasing cost
+        const int tile = a.tiles[4 * ti + 3];                 // tiles in decreasing cost
         const int4 tl = *(const int4 *)(a.tiles + 4 * tile);
         const bool shared = tl.x == a.E;
         const uint8_t *blob = shared ? a.shared : a.experts + (uint64_t)tl.x * a.stride;
-        const uint8_t *w0 = blob + (uint64_t)(fg * kWsRows + 16 * w) * rowb;
-        const uint32_t up_off = (uint32_t)(shared ? a.sh_gate_size : a.gate_size);
+        const uint8_t *w0 = blob + (uint64_t)(fg * 32 * NW + 32 * w) * rowb;
+        const uint64_t up_off = shared ? a.sh_gate_size : a.gate_size;
         const int p0 = tl.y, n = tl.z, nb = (n + 15) >> 4;
         const int tok = a.pair_tok[p0 + min(lane, n - 1)];    // token of tile row lane
         if (w == 0) s_exp[lane] = a.xexp[tok];
-        // step q: this wave's weights, then the token rows and their sub-block sums
         auto issue_w = [&](int q) {
 #pragma unroll
-            for (int i = 0; i < kGbPieces; i++) {   // piece i, lane l: byte o = 1024 i + 16 l of [gate | up],
-                // row (o mod 2304) / 144; lanes past the step's bytes re-read its last 16
-                const uint32_t o = min(i * 1024u + lane * 16u, kGbW - 16);
-                const uint32_t oo = o < kGbHalf ? o : o - kGbHalf;
-                const uint32_t off = (oo / 144) * rowb + oo % 144 + (o >= kGbHalf ? up_off : 0u) + 144u * q;
-                __builtin_amdgcn_global_load_lds((const void *)(w0 + off),
+            for (int i = 0; i < 9; i++) {
+                const uint32_t o = 1024 * i + 16 * lane, r = o / 144;
+                const uint8_t *src = w0 + (r < 32 ? (uint64_t)0 : up_off - 32 * (uint64_t)rowb) + (uint64_t)(r * rowb + o % 144 + 144 * q);
+                __builtin_amdgcn_global_load_lds((const void *)src,
                                                  (__attribute__((address_space(3))) void *)(wb + i * 1024), 16, 0, 0);
             }
         };
         auto issue_x = [&](int q) {
-            for (int q2 = w; q2 < 8 * nb; q2 += kWsWaves) {      // two token rows per wave instruction
-                // 16-byte chunk 8 kg + 4 h + c of a row (lane group kg's values of MFMA (c, h)) lies at
-                // slot (4 (4 h + c) + kg) ^ (row & 15): the 16-lane groups of a 16-byte LDS read then
-                // touch 16 different bank groups
-                const int m = 2 * q2 + (lane >> 5), sl = (lane & 31) ^ (m & 15), c = ((sl & 3) << 3) | (sl >> 2);
-                const uint16_t *src = a.x16 + (uint64_t)__builtin_amdgcn_ds_bpermute(4 * m, tok) * H + q * kGbKC + 8 * c;
+            for (int q2 = w; q2 < 8 * nb; q2 += NW) {          // two token rows per wave instruction
+                const int m = 2 * q2 + (lane >> 5);
+                const uint16_t *src = a.x16 + (uint64_t)__builtin_amdgcn_ds_bpermute(4 * m, tok) * H + q * 256 + 8 * q4_token_chunk(lane, m);
                 __builtin_amdgcn_global_load_lds((const void *)src,
-                                                 (__attribute__((address_space(3))) void *)(ab + 2 * q2 * kGbKC), 16, 0, 0);
+                                                 (__attribute__((address_space(3))) void *)(gu_lds + q2 * 1024), 16, 0, 0);
             }
-            if (w < nb)                                          // the sums of token block w
+            if (w < nb)                                        // the sums of token block w
                 __builtin_amdgcn_global_load_lds(
                     (const void *)(a.xsum + ((uint64_t)__builtin_amdgcn_ds_bpermute(4 * (16 * w + (lane >> 2)), tok) * NQ + q) * 32 + 8 * (lane & 3)),
-                    (__attribute__((address_space(3))) void *)(sb + w * 1024), 16, 0, 0);
+                    (__attribute__((address_space(3))) void *)(gu_lds + kGuA + w * 1024), 16, 0, 0);
         };
         auto run = [&](auto NBC) {
             constexpr int NB = decltype(NBC)::value;
-            f32x4 gA[NB], uA[NB];
+                        f32x4 acc[4][NB];                                  // gate rows 0..15, 16..31, up rows 0..15, 16..31
 #pragma unroll
-            for (int b = 0; b < NB; b++) { gA[b] = (f32x4){0.f, 0.f, 0.f, 0.f}; uA[b] = gA[b]; }
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int tb = 0; tb < NB; tb++) acc[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
             for (int q = 0; q < NQ; q++) {
                 issue_w(q);
                 issue_x(q);
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();                               // everyone's loads of step q have landed
-                // Lane group kg owns sub-blocks 2 kg and 2 kg + 1 of the super-block
-                // (MFMA (c, h): lane group kg's 8 values are values 8c..8c+7 of
-                // sub-block 2 kg + h; the token operand is read in the same
-                // order), so each lane decodes two scales instead of all eight.
-                // NM matrices together share every token operand read.
-                auto pass = [&](auto NMC, const uint8_t *rw, auto &...accs) {
-                    constexpr int NM = decltype(NMC)::value;
-                    f32x4 *acc[NM] = {&accs[0]...};
-                    f16x2 sp[NM][2];
-                    f32x4 dd[NM][NB];
-#pragma unroll
-                    for (int g = 0; g < NM; g++) {
-                        q4_scale_pair(*(const uint4 *)(rw + g * kGbHalf), kg, sp[g]);
-#pragma unroll
-                        for (int tb = 0; tb < NB; tb++) dd[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                    }
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        f16x8 bw[NM][2];
-#pragma unroll
-                        for (int g = 0; g < NM; g++)   // 8 bytes of codes: sub-blocks 2 kg, 2 kg + 1
-                            q4_codes_f16(*(const uint2 *)(rw + g * kGbHalf + 16 + 32 * kg + 8 * c), sp[g], bw[g][0], bw[g][1]);
-#pragma unroll
-                        for (int h = 0; h < 2; h++)
-#pragma unroll
-                            for (int tb = 0; tb < NB; tb++) {
-                                const f16x8 av = *(const f16x8 *)((const uint8_t *)ab + aoff[c] + 256 * h + 8192 * tb);
-#pragma unroll
-                                for (int g = 0; g < NM; g++)
-                                    dd[g][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw[g][h], dd[g][tb], 0, 0, 0);
-                            }
-                        if constexpr (NB > 2) __builtin_amdgcn_sched_barrier(0);
-                    }
-                    f16x8 mn[NM];
-                    float d[NM], dm[NM];
-#pragma unroll
-                    for (int g = 0; g < NM; g++) {
-                        const uint4 hw = *(const uint4 *)(rw + g * kGbHalf);
-                        mn[g] = q4_mins_f16(hw);
-                        d[g] = h2f(hw.x) * 16384.f;              // codes entered times 2^-14
-                        dm[g] = h2f(hw.x >> 16) * -32.f;         // sums entered divided by 32
-                    }
-#pragma unroll
-                    for (int tb = 0; tb < NB; tb++) {
-                        // A: the sums of token 16 tb + col: hi, mid, lo terms of the eight sub-blocks, zeros
-                        const f16x8 sa = *(const f16x8 *)(sb + (16 * tb + col) * 64 + 16 * kg);
-#pragma unroll
-                        for (int g = 0; g < NM; g++) {
-                            const f32x4 ms = __builtin_amdgcn_mfma_f32_16x16x32_f16(sa, mn[g], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                acc[g][tb][i] = fmaf(d[g], dd[g][tb][i], fmaf(dm[g], ms[i], acc[g][tb][i]));
-                        }
-                    }
-                };
-                if constexpr (NB <= 2) {
-                    pass(std::integral_constant<int, 2>{}, wb + col * 144, gA, uA);
-                } else {
-                    pass(std::integral_constant<int, 1>{}, wb + col * 144, gA);
-                    pass(std::integral_constant<int, 1>{}, wb + kGbHalf + col * 144, uA);
-                }
+                q4_super_block<4, NB>(acc, wb + col * 144, kGuHalf, gu_lds, aoff, sb, col, kg);
                 __syncthreads();                               // the step's LDS is free for the next one
             }
-            const int row = fg * kWsRows + 16 * w + col;
 #pragma unroll
-            for (int tb = 0; tb < NB; tb++) {
+            for (int g = 0; g < 2; g++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int m = 16 * tb + 4 * kg + i;
-                    if (m < n) {
-                        const int sx = s_exp[m];
-                        const float g = ldexpf(gA[tb][i], sx), u = ldexpf(uA[tb][i], sx);
-                        const float val = (g / (1.0f + expf(-g))) * u;
-                        const __bf16 hi = (__bf16)val;
-                        const __bf16 lo = (__bf16)(val - (float)hi);
-                        const uint64_t o = (uint64_t)(p0 + m) * a.F + row;
-                        a.act_hi[o] = __builtin_bit_cast(uint16_t, hi);
-                        a.act_lo[o] = __builtin_bit_cast(uint16_t, lo);
-                    }
-                }
-            }
+                for (int tb = 0; tb < NB; tb++)
+                    q4_finish(a, s_exp, p0, n, fg * 32 * NW + 32 * w + 16 * g, acc[g][tb], acc[2 + g][tb], tb, col, kg);
         };
         switch (nb) {
             case 1: run(std::integral_constant<int, 1>{}); break;
@@ -1221,7 +1238,10 @@ __global__ __launch_bounds__(64 * kWsWaves, 4) void k_pf_gateup_f16(PrefillArgs 
             case 3: run(std::integral_constant<int, 3>{}); break;
             default: run(std::integral_constant<int, 4>{}); break;
         }
-        __syncthreads();                                       // s_item and s_exp are free
+        if (tid == 0) s_item = gridDim.x + atomicAdd(a.n_tiles + 2, 1);
+        __syncthreads();                                       // s_exp and the LDS are free
+        item = s_item;
+        __syncthreads();
     }
 }
 
@@ -1864,13 +1884,13 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
         static bool gb_attr = false;   // above the 64 KiB default of dynamic LDS
         if (!gb_attr) {
             hipError_t e = hipFuncSetAttribute((const void *)k_pf_gateup_f16,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGbLds);
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGuLds);
             if (e != hipSuccess) return e;
             gb_attr = true;
         }
         int dev = 0, n_cu = 256;
         if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-        k_pf_gateup_f16<<<2 * n_cu, 64 * kWsWaves, kGbLds, s>>>(a);
+        k_pf_gateup_f16<<<2 * n_cu, 64 * kGuWaves, kGuLds, s>>>(a);
         err = hipGetLastError();
     }
 #define FO_GU(G, U) if (a.gate_type == G && a.up_type == U) err = launch_gateup_t<G, U>(a, s);
