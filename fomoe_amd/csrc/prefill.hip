@@ -1659,13 +1659,18 @@ __global__ __launch_bounds__(64 * kPfThinWaves) void k_pf_down_thin(PrefillArgs 
     uint8_t *zero = sx + kPfThin * kPfThinX;
     uint8_t *tb = zero + kPfThinZero + wv * kPfThinTile;
     const int n_thick = a.n_tiles[1], n_thin = a.n_tiles[0] - n_thick;
-    const int upt = a.H / kPfThinUnitRows, nunits = n_thin * upt;
+    // 8 tiles per wave and unit where that fills the grid twice, else 4 or 2: few thin
+    // experts otherwise leave work-groups with one long unit or none (16 tokens, 49
+    // thin experts: 59 -> 42 us; at 512 tokens 8 tiles stay the fastest)
+    int tpw = kPfThinTPW;
+    while (tpw > 2 && n_thin * (a.H / (16 * kPfThinWaves * tpw)) < 2 * (int)gridDim.x) tpw >>= 1;
+    const int urows = 16 * kPfThinWaves * tpw, upt = a.H / urows, nunits = n_thin * upt;
     if ((int)threadIdx.x < kPfThinZero / 16) *(uint4 *)(zero + 16 * threadIdx.x) = make_uint4(0, 0, 0, 0);
     const int r = lane & 15, g = lane >> 4, n = g >> 1, j = g & 1, L = r & 3;
     const bool valid = (r >> 2) == g && L < 3;
     const uint32_t aoff = (8 * n + j) * 48 + 16 * L, soff = limb_bytes + (8 * n + j) * 8;
     for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-        const int ti = n_thick + u / upt, row0 = (u % upt) * kPfThinUnitRows + wv * 16 * kPfThinTPW;
+        const int ti = n_thick + u / upt, row0 = (u % upt) * urows + wv * 16 * tpw;
         const int tile = a.tiles[4 * ti + 3];
         const int4 t4 = *(const int4 *)(a.tiles + 4 * tile);
         const bool shared = t4.x == a.E;
@@ -1702,10 +1707,10 @@ __global__ __launch_bounds__(64 * kPfThinWaves) void k_pf_down_thin(PrefillArgs 
             if (lane == 0) s_pe[wv] = a.pexp[p0 + wv];
         }
         __syncthreads();
-        for (int tt = 0; tt < kPfThinTPW; tt++) {
+        for (int tt = 0; tt < tpw; tt++) {
 #pragma unroll
             for (int i = 0; i < NV; i++) *(uint4 *)(tb + min(i * 1024u + lane * 16u, kPfThinTile - 16)) = v[i];
-            if (tt + 1 < kPfThinTPW) issue(tt + 1);
+            if (tt + 1 < tpw) issue(tt + 1);
             Q6kSlot qs[4];
 #pragma unroll
             for (int b = 0; b < 4; b++) q6k_slot_load(qs[b], tb + r * rb + b * 210, n, j);
