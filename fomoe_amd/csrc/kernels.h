@@ -26,6 +26,9 @@ struct MatvecArgs {
 // MatvecArgs::xf (no separate activation-prep launch): the Q6_K tile-staged
 // kernel always, the general kernel when every matrix shares one x.
 bool matvec_self_prep(int type, uint64_t row_bytes, int K, uint64_t x_stride);
+// True when, for shapes matvec_self_prep declines because every matrix has its
+// own x, the general kernel can still prepare them itself.
+bool matvec_preps_each(int type, int M, int K, int n_mats, int n_cu);
 
 // Router: logits = W_r . h (+ bias), h = rms_norm(x)*w when norm_w != NULL,
 // then (last work-group) softmax, top-k with lowest-index ties, renormalise,

@@ -131,16 +131,32 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     L.init(lane, S);
     XRegs<T, U> X;
     int64_t cur = -1;
-    // With a shared fp32 x (xf, xf_stride 0) the work-group prepares it in LDS
-    // itself (one thread per group, bit-identical to k_xprep); otherwise x
-    // comes prepared from global memory.
+    // With fp32 x (xf) the work-group prepares it in LDS itself (one thread per
+    // group, bit-identical to k_xprep): the one all matrices share (xf_stride
+    // 0), or those of the at most two matrices its waves' consecutive tasks lie
+    // in (matvec_preps_each); otherwise x comes prepared from global memory.
     extern __shared__ __attribute__((aligned(16))) uint8_t xs_lds[];
     const uint8_t *xq = a.xq;
+    uint64_t xstep = a.x_stride;
+    int64_t m0 = 0;
     if (a.xf) {
         constexpr int GSZ = Fmt<T>::GSZ;
         const int ng = a.K / GSZ;
-        for (int g = threadIdx.x; g < ng; g += blockDim.x)
-            prep_group<GSZ>(a.xf + g * GSZ, xs_lds + g * (kLimbs * GSZ), xs_lds + xq_limb_bytes(a.K) + g * 8);
+        int nx = 1;
+        if (a.xf_stride) {
+            const int w0 = (int)(blockIdx.x * (blockDim.x >> 6));
+            int64_t f0, f1, l0, l1;
+            wave_share(tpm * a.n_mats, w0, nw, f0, f1);
+            wave_share(tpm * a.n_mats, w0 + (int)(blockDim.x >> 6) - 1, nw, l0, l1);
+            m0 = min(f0 / tpm, (int64_t)a.n_mats - 1);
+            nx = l1 > f0 ? (int)((l1 - 1) / tpm - m0) + 1 : 1;
+            xstep = lds_round(xq_bytes(a.K, GSZ));
+        }
+        for (int i = threadIdx.x; i < ng * nx; i += blockDim.x) {
+            const int v = i / ng, g = i - v * ng;
+            uint8_t *xv = xs_lds + v * xstep;
+            prep_group<GSZ>(a.xf + (m0 + v) * a.xf_stride + g * GSZ, xv + g * (kLimbs * GSZ), xv + xq_limb_bytes(a.K) + g * 8);
+        }
         __syncthreads();
         xq = xs_lds;
     }
@@ -158,7 +174,7 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     for (int64_t t = t0; t < t1; t++) {
         const int64_t m = t / tpm;
         const int rb = (int)(t - m * tpm);
-        if (m != cur && (cur < 0 || a.x_stride)) X.load(L, xq + m * a.x_stride, a.K);
+        if (m != cur && (cur < 0 || xstep)) X.load(L, xq + (m - m0) * xstep, a.K);
         cur = m;
         const uint8_t *W = a.W + m * a.mat_stride;
         RowRaw<T, U> raw[R];
@@ -198,6 +214,11 @@ static bool geometry(int type, int K, int &G, int &U) {
     return true;
 }
 
+static bool geometry_ok(int type, int K) {
+    int G, U;
+    return geometry(type, K, G, U);
+}
+
 static int waves_for(int64_t tasks, int n_cu, int per_cu) {
     const int64_t cap = (int64_t)n_cu * per_cu;
     return (int)(tasks < cap ? (tasks > 0 ? tasks : 1) : cap);
@@ -210,7 +231,7 @@ static hipError_t matvec_t(const MatvecArgs &a, hipStream_t s, int n_cu) {
     const int P = 64 / G;
     const int64_t tasks = (int64_t)((a.M + P * R - 1) / (P * R)) * a.n_mats;
     const int blocks = (waves_for(tasks, n_cu, 16) + 3) / 4;
-    const size_t lds = a.xf ? lds_round(xq_bytes(a.K, Fmt<T>::GSZ)) : 0;
+    const size_t lds = a.xf ? lds_round(xq_bytes(a.K, Fmt<T>::GSZ)) * (a.xf_stride ? 2 : 1) : 0;
 #define FO_MV(GG, UU) \
     if (G == GG && U == UU) { k_matvec<T, UU, GG, R><<<blocks, 256, lds, s>>>(a); return hipGetLastError(); }
     FO_MV(64, 1) FO_MV(64, 2) FO_MV(64, 3) FO_MV(64, 4)
@@ -766,6 +787,30 @@ static bool tile_shape(int type, uint64_t row_bytes, int K) {
     return false;
 }
 
+// Launches of less weight than this run on the general kernel, whose grid of
+// two-row tasks spreads a small batch over the chip where a tile kernel's waves
+// (16 rows each, several tiles one after the other) leave most of it idle. Per
+// launch at 1024 / 4096 / 8192 rows (general against tile kernel, us): Q4_K K
+// 4096 5.1 / 6.3 / 8.5 against 7.8 / 8.2 / 8.7; Q6_K K 1024 4.6 / 4.8 / 5.4
+// against 8.6 / 8.9 / 9.0; Q8_0 K 4096 5.8 / 8.8 / 13.6 against 15.0 / 15.3 /
+// 15.8. The two meet between 18 MB (Q8_0, K 1024) and 75 MB (Q4_K, K 8192).
+constexpr uint64_t kSmallBytes = 16u << 20;
+static bool small_launch(const MatvecArgs &a) {
+    return a.xf && (a.xf_stride == 0 || a.n_mats == 1) && (uint64_t)a.M * a.n_mats * a.row_bytes < kSmallBytes;
+}
+
+// Whether the general kernel prepares the separate x of every matrix itself: a
+// work-group's four waves then lie in at most two matrices (their tasks are no
+// more than one matrix has), and two prepared vectors fit the default LDS.
+bool matvec_preps_each(int type, int M, int K, int n_mats, int n_cu) {
+    int G, U;
+    if (!geometry(type, K, G, U)) return false;
+    const int rows = 64 / G * 2;   // matvec_t's R = 2
+    const int64_t tpm = (M + rows - 1) / rows, tasks = tpm * n_mats;
+    const int64_t nw = ((int64_t)waves_for(tasks, n_cu, 16) + 3) / 4 * 4;
+    return 4 * ((tasks + nw - 1) / nw) <= tpm && 2 * lds_round(xq_bytes(K, gsz_of(type))) <= 62 * 1024;
+}
+
 bool matvec_self_prep(int type, uint64_t row_bytes, int K, uint64_t x_stride) {
     if (type == GGML_TYPE_Q6_K && row_bytes == (uint64_t)K / 256 * 210 && K % 256 == 0 && K <= 1024)
         return true;   // tile-staged kernel: one matrix per work-group, any x_stride
@@ -776,6 +821,18 @@ bool matvec_self_prep(int type, uint64_t row_bytes, int K, uint64_t x_stride) {
 
 hipError_t launch_matvec(int type, const MatvecArgs &a, hipStream_t s, int n_cu) {
     if (a.M <= 0 || a.n_mats <= 0) return hipErrorInvalidValue;
+    if (small_launch(a) && geometry_ok(type, a.K)) {
+        MatvecArgs b = a;
+        b.xf_stride = 0;   // one x
+        switch (type) {
+            case GGML_TYPE_Q4_K: return matvec_t<GGML_TYPE_Q4_K, 2>(b, s, n_cu);
+            case GGML_TYPE_Q5_K: return matvec_t<GGML_TYPE_Q5_K, 2>(b, s, n_cu);
+            case GGML_TYPE_Q6_K: return matvec_t<GGML_TYPE_Q6_K, 2>(b, s, n_cu);
+            case GGML_TYPE_Q8_0: return matvec_t<GGML_TYPE_Q8_0, 2>(b, s, n_cu);
+            case GGML_TYPE_MXFP4: return matvec_t<GGML_TYPE_MXFP4, 2>(b, s, n_cu);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (type) {
         case GGML_TYPE_Q4_K:
             if (a.xf && tile_shape(type, a.row_bytes, a.K)) {   // tile-staged path

@@ -213,6 +213,28 @@ def test_matvec_batched(gpu, t, M, K, per_x):
         assert parity_err(got[m], want) <= TOL, m
 
 
+@pytest.mark.parametrize("t,M,K,n,per_x", [
+    # either side of the 16 MiB below which a launch with one x runs on the general kernel
+    (O.Q4_K, 1024, 4096, 7, False), (O.Q4_K, 1024, 4096, 8, False), (O.Q6_K, 4096, 1024, 4, False),
+    (O.Q6_K, 4096, 1024, 5, False), (O.Q8_0, 17, 1024, 1, True),
+    # separate x on the general kernel: work-groups inside one matrix, across two (odd
+    # task counts), and matrices too small for that (prepared by a launch of their own)
+    (O.Q5_K, 1000, 2816, 3, True), (O.Q5_K, 37, 2816, 7, True), (O.Q6_K, 61, 2048, 50, True),
+    (O.Q8_0, 33, 96, 40, True), (O.Q4_K, 1, 512, 3, True), (O.Q6_K, 9, 16384, 2, True)])
+def test_matvec_general_routes(gpu, t, M, K, n, per_x):
+    say("matvec routes", t, M, K, n, per_x)
+    stride = O.row_bytes(t, K) * M
+    W = np.concatenate([O.synth_quant(t, 18, 100 + m, 0.02, M, K) for m in range(n)]) if K % 256 == 0 else \
+        np.random.default_rng(5).integers(0, 60, stride * n).astype(np.uint8)   # (the generator takes K % 256 == 0)
+    xs = np.stack([O.synth_f32(19, m if per_x else 0, 1.0, K) for m in range(n)])
+    dW, dx, dy = gpu.upload(W), gpu.upload(xs if per_x else xs[0]), gpu.alloc(4 * M * n)
+    gpu.matvec_batched(t, dW, stride, n, dx, K if per_x else 0, dy, M, M, K)
+    got = gpu.download(dy, np.float32, M * n).reshape(n, M)
+    for m in range(n):
+        want = O.mat_vec(t, W[m * stride:(m + 1) * stride], xs[m], M, K)
+        assert parity_err(got[m], want) <= TOL, m
+
+
 # ------------------------------------------------------------------ router
 @pytest.mark.parametrize("norm,bias", [(False, False), (True, True)])
 def test_router_topk(gpu, norm, bias):
