@@ -87,6 +87,7 @@ void gpu_free(gpu_ctx_t *c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
+    delete c->stage;
     void *bufs[] = {c->logits, c->counter, c->ids, c->weights, c->xq_h, c->xq_act, c->act,
                     c->act2, c->vec_in, c->vec_out, c->staging, c->pf_logits, c->pf_ids,
                     c->pf_w, c->pf_pairpos, c->pf_pairtok, c->pf_tiles, c->pf_ntiles,
@@ -600,10 +601,26 @@ int gpu_expert_ffn(gpu_ctx_t *ctx, const float *h, void **expert_buffers, const 
     if (hipMemcpyAsync(ctx->vec_in, h, sizeof(float) * H, hipMemcpyHostToDevice, s) != hipSuccess)
         return -1;
     for (int e = 0; e < n; e++)
-        if (!expert_buffers[e] ||
-            hipMemcpyAsync(ctx->staging + (size_t)e * stride, expert_buffers[e], stride,
-                           hipMemcpyHostToDevice, s) != hipSuccess)
+        if (!expert_buffers[e]) return -1;
+    // the blobs: through the pinned ring where they fill at least one slot of
+    // it (82 MB: 1.81 ms a call against 2.93 with plain copies)
+    const uint64_t blob_bytes = (uint64_t)n * stride;
+    const bool staged = blob_bytes >= HostStage::kSlot && blob_bytes <= HostStage::kMaxBytes;
+    if (staged && !ctx->stage_tried) {
+        ctx->stage_tried = true;
+        ctx->stage = HostStage::create();
+    }
+    if (staged && ctx->stage) {
+        if (ctx->stage->run(expert_buffers, n, stride, ctx->staging, s) != hipSuccess) {
+            (void)hipStreamSynchronize(s);
             return -1;
+        }
+    } else {
+        for (int e = 0; e < n; e++)
+            if (hipMemcpyAsync(ctx->staging + (size_t)e * stride, expert_buffers[e], stride,
+                               hipMemcpyHostToDevice, s) != hipSuccess)
+                return -1;
+    }
     if (hipMemcpyAsync(ctx->weights, scores, sizeof(float) * n, hipMemcpyHostToDevice, s) != hipSuccess)
         return -1;
     const uint64_t rb_g = fomoe_row_bytes(gate_type, H), rb_u = fomoe_row_bytes(up_type, H);

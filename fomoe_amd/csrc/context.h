@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "gpu.h"
+#include "host_stage.h"
 
 struct gpu_ctx {
     int device = 0;
@@ -59,6 +60,10 @@ struct gpu_ctx {
     // pinned staging for host->device uploads of expert stores
     uint8_t *pin[2] = {nullptr, nullptr};
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
+
+    // pageable-to-device copies of gpu_expert_ffn (made by the first call large enough)
+    HostStage *stage = nullptr;
+    bool stage_tried = false;
 
     // values given to gpu_set_{ram,vram}_cache_mb (recorded; no cache tiers here)
     int ram_cache_mb = -1, vram_cache_mb = -1;

@@ -235,6 +235,33 @@ def test_matvec_general_routes(gpu, t, M, K, n, per_x):
         assert parity_err(got[m], want) <= TOL, m
 
 
+@pytest.mark.parametrize("n,pad", [(2, 0), (5, 1001), (10, 37)])
+def test_expert_ffn_staged_copies(gpu, n, pad):
+    """Blobs through the pinned ring (8 MiB and more in all): slots that end
+    inside a blob, blobs of odd size, more slots than the ring has, and a second
+    call with other blobs right behind the first; against the same experts one
+    per call (each below a slot: plain copies)."""
+    say("expert_ffn staged", n, pad)
+    H, F = 4096, 1024
+    gs, ds = O.row_bytes(O.Q4_K, H) * F, O.row_bytes(O.Q6_K, F) * H
+    size = 2 * gs + ds
+    d = gpu.alloc(size * n)
+    for call in range(2):
+        for k, off, t, M, K in ((0, 0, O.Q4_K, F, H), (1, gs, O.Q4_K, F, H), (2, 2 * gs, O.Q6_K, H, F)):
+            gpu.synth_quant(t, 40 + call, k, 16, 0.02, M, K, n, d.offset(off), size)
+        blobs = [np.concatenate([b, np.full(pad, 0xA5, np.uint8)])
+                 for b in gpu.download(d, np.uint8, size * n).reshape(n, size)]
+        h, w = O.synth_f32(41 + call, 0, 1.0, H), np.linspace(0.3, 1.0, n).astype(np.float32)
+        rc, out = gpu.expert_ffn(h, blobs, w, H, F, gs, gs, size + pad, O.Q4_K, O.Q4_K, O.Q6_K)
+        assert rc == 0
+        ref = np.zeros(H, np.float64)
+        for e in range(n):
+            rc, one = gpu.expert_ffn(h, blobs[e:e + 1], w[e:e + 1], H, F, gs, gs, size + pad, O.Q4_K, O.Q4_K, O.Q6_K)
+            assert rc == 0
+            ref += one
+        assert inf_rel(out, ref) < 1e-6   # n fp32 additions of the same terms
+
+
 # ------------------------------------------------------------------ router
 @pytest.mark.parametrize("norm,bias", [(False, False), (True, True)])
 def test_router_topk(gpu, norm, bias):
