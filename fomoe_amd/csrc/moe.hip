@@ -182,6 +182,21 @@ hipError_t launch_route(const RouteArgs &a, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
+// The first `rounds` selections of one wave, with the values per lane that E
+// needs: one or two by arg-max rounds, more by the threshold ranking.
+FO_DEV void select_experts(const ExpandArgs &a, int rounds, bool full, int *s_ids, float *s_w, float2 *s_cand, float *s_val) {
+    float *w = full ? s_w : nullptr;
+    if (rounds <= 2) {
+        if (a.E <= 128) wave_topk<2>(a.logits, a.E, rounds, s_ids, w);
+        else if (a.E <= 512) wave_topk<8>(a.logits, a.E, rounds, s_ids, w);
+        else wave_topk<16>(a.logits, a.E, rounds, s_ids, w);
+    } else {
+        if (a.E <= 128) wave_topk_thr<2>(a.logits, a.E, rounds, s_ids, w, s_cand, s_val);
+        else if (a.E <= 512) wave_topk_thr<8>(a.logits, a.E, rounds, s_ids, w, s_cand, s_val);
+        else wave_topk_thr<16>(a.logits, a.E, rounds, s_ids, w, s_cand, s_val);
+    }
+}
+
 // ============================================================ K2: expand
 // One work-group of TR/RW waves per task (expert slot e, block of TR rows, TR
 // = the activation-group size of the down projection; RW rows per wave); the
@@ -225,14 +240,7 @@ __global__ __launch_bounds__((ExpandShape<T, TR, U>::THREADS), 3) void k_expand(
     const bool full = a.shared ? (e == a.k && rb == 0) : blockIdx.x == 0;
     const int rounds = full ? a.k : (routed ? e + 1 : 0);
     if (wv == 0 && rounds > 0) {
-        // one or two selections: arg-max rounds; more: the threshold ranking
-        if (rounds <= 2) {
-            if (a.E <= 512) wave_topk<8>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr);
-            else wave_topk<16>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr);
-        } else {
-            if (a.E <= 512) wave_topk_thr<8>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr, s_cand, s_val);
-            else wave_topk_thr<16>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr, s_cand, s_val);
-        }
+        select_experts(a, rounds, full, s_ids, s_w, s_cand, s_val);
         if (full && lane < a.k) { a.ids[lane] = s_ids[lane]; a.weights[lane] = s_w[lane]; }
     }
     stage_lds_wait();
@@ -321,14 +329,7 @@ __global__ __launch_bounds__(256, 3) void k_expand_q4t(ExpandArgs a) {
     const bool full = a.shared ? (e == a.k && rb == 0) : blockIdx.x == 0;
     const int rounds = full ? a.k : (routed ? e + 1 : 0);
     if (wv == 0 && rounds > 0) {
-        // one or two selections: arg-max rounds; more: the threshold ranking
-        if (rounds <= 2) {
-            if (a.E <= 512) wave_topk<8>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr);
-            else wave_topk<16>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr);
-        } else {
-            if (a.E <= 512) wave_topk_thr<8>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr, s_cand, s_val);
-            else wave_topk_thr<16>(a.logits, a.E, rounds, s_ids, full ? s_w : nullptr, s_cand, s_val);
-        }
+        select_experts(a, rounds, full, s_ids, s_w, s_cand, s_val);
         if (full && lane < a.k) { a.ids[lane] = s_ids[lane]; a.weights[lane] = s_w[lane]; }
     }
     stage_lds_wait();
@@ -629,7 +630,6 @@ static hipError_t reduce_tile(const ReduceArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_reduce(int type, const ReduceArgs &a, hipStream_t s, int n_cu) {
-    (void)n_cu;
     const int slot = type == GGML_TYPE_Q8_0 ? 32 : 64;
     const int n_tot = a.k + (a.shared ? 1 : 0);
     if (a.F % slot || a.F / slot > 64 || a.k <= 0 || n_tot > 16 || a.H <= 0) return hipErrorInvalidValue;
@@ -645,15 +645,21 @@ hipError_t launch_reduce(int type, const ReduceArgs &a, hipStream_t s, int n_cu)
         if (type == GGML_TYPE_Q5_K) return reduce_tile<GGML_TYPE_Q5_K, 16, 704>(a, s);
     }
     if (a.act_f32) return hipErrorInvalidValue;   // only the LDS-staged kernel prepares from fp32
-    constexpr int RP = 4;
+    // passes of 64 / G rows per wave: fewer where four of them leave CUs without
+    // a work-group (H = 2048, F = 768, 8 experts:
+    // 5.7 us with two passes and 256 work-groups, 7.7 with four, 7.3 with one)
+    int RP = 4;
+    while (RP > 1 && (a.H + 64 / G * RP - 1) / (64 / G * RP) < n_cu) RP >>= 1;
     const int RB = (64 / G) * RP;
     const int grid = (a.H + RB - 1) / RB;
     const int threads = 64 * n_tot;
-#define FO_K3(TT, GG) \
-    if (type == TT && G == GG) { k_reduce<TT, GG, RP><<<grid, threads, 0, s>>>(a); return hipGetLastError(); }
-#define FO_K3T(TT) FO_K3(TT, 64) FO_K3(TT, 32) FO_K3(TT, 16) FO_K3(TT, 8) FO_K3(TT, 4)
+#define FO_K3(TT, GG, RR) \
+    if (type == TT && G == GG && RP == RR) { k_reduce<TT, GG, RR><<<grid, threads, 0, s>>>(a); return hipGetLastError(); }
+#define FO_K3G(TT, GG) FO_K3(TT, GG, 4) FO_K3(TT, GG, 2) FO_K3(TT, GG, 1)
+#define FO_K3T(TT) FO_K3G(TT, 64) FO_K3G(TT, 32) FO_K3G(TT, 16) FO_K3G(TT, 8) FO_K3G(TT, 4)
     FO_K3T(GGML_TYPE_Q4_K) FO_K3T(GGML_TYPE_Q5_K) FO_K3T(GGML_TYPE_Q6_K) FO_K3T(GGML_TYPE_Q8_0)
 #undef FO_K3T
+#undef FO_K3G
 #undef FO_K3
     return hipErrorInvalidValue;
 }

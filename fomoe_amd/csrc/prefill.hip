@@ -293,7 +293,8 @@ __global__ __launch_bounds__(256) void k_pf_topk(PrefillArgs a) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= a.T) return;
     const int K1 = a.k + 1;
-    if (a.E <= 512) wave_topk<8>(a.logits + (uint64_t)t * a.E, a.E, a.k, a.ids + (uint64_t)t * a.k, a.w + (uint64_t)t * K1);
+    if (a.E <= 128) wave_topk<2>(a.logits + (uint64_t)t * a.E, a.E, a.k, a.ids + (uint64_t)t * a.k, a.w + (uint64_t)t * K1);
+    else if (a.E <= 512) wave_topk<8>(a.logits + (uint64_t)t * a.E, a.E, a.k, a.ids + (uint64_t)t * a.k, a.w + (uint64_t)t * K1);
     else wave_topk<16>(a.logits + (uint64_t)t * a.E, a.E, a.k, a.ids + (uint64_t)t * a.k, a.w + (uint64_t)t * K1);
     float sw = 1.f;
     if (a.shared_gate_vec) {

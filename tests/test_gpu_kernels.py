@@ -354,6 +354,29 @@ def test_moe_layer_norm_residual_gate(gpu):
     assert np.array_equal(got, (x + ffn).astype(np.float32))
 
 
+@pytest.mark.parametrize("H,F,E,k", [(4096, 768, 16, 3), (2048, 768, 128, 8), (1024, 768, 129, 8), (512, 256, 128, 16),
+                                     (1536, 1280, 127, 2)])
+def test_moe_layer_small_grids(gpu, H, F, E, k):
+    """The general down kernel with four, two and one passes per wave (its
+    grid against the CU count; 1280: more lanes per row, fewer rows), and the
+    selection with 2 values per lane up to 128 experts: routing and outputs
+    against the fp32 oracle."""
+    from fomoe_amd import synthetic as S
+    say(f"layer small grids H={H} F={F} E={E} k={k}")
+    shape = S.LayerShape(n_embd=H, inter=F, n_experts=E, k=k, shared=False)
+    L = S.build_layer(gpu, shape, 0, seed=73, zipf_s=1.1, norm=False)
+    h = O.synth_f32(74, 0, 1.0, H)
+    dh, dout = gpu.upload(h), gpu.alloc(4 * H)
+    gpu.moe_layer(L.desc, dh, dout, 0)
+    got = gpu.download(dout, np.float32, H)
+    ids, w, _ = gpu.last_routing(k)
+    d, keep = _prefill_host_layer(shape, 0, 73, True, experts_needed=list(ids))
+    want, oi, ow = O.moe_layer(d, h, 0)
+    assert np.array_equal(ids, oi)
+    assert inf_rel(w, ow) < 1e-5
+    assert inf_rel(got, want) < 1e-5
+
+
 @pytest.mark.parametrize("E,H", [(1, 512), (15, 1024), (16, 512), (1023, 8192)])
 def test_route_gate_vector(gpu, E, H):
     """The shared-expert gate as the router kernel's work-group of its own,
