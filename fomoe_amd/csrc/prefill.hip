@@ -904,8 +904,8 @@ __global__ __launch_bounds__(kPfGateWaves * 64, 4) void k_pf_gateup(PrefillArgs 
 // work-groups share a CU, and the loads of one overlap the arithmetic of the
 // other. Work-groups take their first item by index and the others from a counter
 // (reset by k_pf_group). What bounds it: the steps' latencies at two waves per
-// SIMD, not a unit (at 512 tokens VALU ~40 %, MFMA ~22 %, LDS ~15 % busy) and,
-// for tiles of few tokens, HBM (1.1 x the distinct bytes fetched). Trace, against
+// SIMD, not a unit (tiles above 16 tokens at 512 tokens: VALU 37 %, MFMA 22 %,
+// LDS 13 % busy) and, for tiles of few tokens, HBM. Trace, against
 // eight waves of 16 + 16 rows: 16 / 512 / 4096 tokens 66 / 331 / 1303 us
 // against 73 / 338 / 1360. Measured slower: one work-group per CU with both
 // operands double-buffered by direct loads (218 / 1466 us at 512 / 4096 tokens
