@@ -401,13 +401,17 @@ FO_DEV void pf_place(const PrefillArgs &a, const uint32_t *bm, const uint32_t *p
 // tables and each (segment, expert)'s first pair slot, k_pf_gplace places the
 // segment's pairs.
 __global__ __launch_bounds__(1024) void k_pf_gcount(PrefillArgs a) {
-    __shared__ int s_cnt[1024];
+    extern __shared__ uint32_t lds[];
+    constexpr int W = kPfSeg / 32, Ws = pf_group_stride(W);
     const int t0 = blockIdx.x * kPfSeg, t1 = min(a.T, t0 + kPfSeg);
-    s_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    for (int i = t0 * a.k + threadIdx.x; i < t1 * a.k; i += 1024) atomicAdd(&s_cnt[a.ids[i]], 1);
-    __syncthreads();
-    if ((int)threadIdx.x < a.E) a.segs[blockIdx.x * a.E + threadIdx.x] = s_cnt[threadIdx.x];
+    // bits, not occurrences: the ranks of a token with non-finite logits may
+    // name one expert several times, and share one slot
+    pf_bitmaps(a, lds, Ws, t0, t1);
+    if ((int)threadIdx.x < a.E) {
+        int cnt = 0;
+        for (int w = 0; w < W; w++) cnt += __popc(lds[threadIdx.x * Ws + w]);
+        a.segs[blockIdx.x * a.E + threadIdx.x] = cnt;
+    }
 }
 
 __global__ __launch_bounds__(1024) void k_pf_gplace(PrefillArgs a) {
@@ -1865,8 +1869,10 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute((const void *)k_pf_group, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            2 * (kPfGroupLds + kMaxE) * (int)sizeof(uint32_t));
         if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute((const void *)k_pf_gplace, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                2 * kMaxE * pf_group_stride(kPfSeg / 32) * (int)sizeof(uint32_t));
+        constexpr int seg = kMaxE * pf_group_stride(kPfSeg / 32) * (int)sizeof(uint32_t);
+        e = hipFuncSetAttribute((const void *)k_pf_gcount, hipFuncAttributeMaxDynamicSharedMemorySize, seg);
+        if (e != hipSuccess) return e;
+        e = hipFuncSetAttribute((const void *)k_pf_gplace, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * seg);
         if (e != hipSuccess) return e;
         lds_attr = true;
     }
@@ -1874,9 +1880,10 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
         k_pf_group<<<1, 1024, 2 * (size_t)a.E * pf_group_stride(W) * sizeof(uint32_t), s>>>(a, 0);
     } else {
         const int n_seg = (a.T + kPfSeg - 1) / kPfSeg;
-        k_pf_gcount<<<n_seg, 1024, 0, s>>>(a);
+        const size_t seg = (size_t)a.E * pf_group_stride(kPfSeg / 32) * sizeof(uint32_t);
+        k_pf_gcount<<<n_seg, 1024, seg, s>>>(a);
         k_pf_group<<<1, 1024, 0, s>>>(a, n_seg);
-        k_pf_gplace<<<n_seg, 1024, 2 * (size_t)a.E * pf_group_stride(kPfSeg / 32) * sizeof(uint32_t), s>>>(a);
+        k_pf_gplace<<<n_seg, 1024, 2 * seg, s>>>(a);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;

@@ -1405,6 +1405,35 @@ def test_prefill_pass_sizes(gpu, E, k, T, cut):
     assert np.array_equal(got, gpu.download(d2, np.uint32, T * H))
 
 
+def test_prefill_segments_nonfinite_tokens(gpu):
+    """Tokens with non-finite logits in a batch above one grouping table: all
+    their ranks may name the same expert, whose pair then has one slot, as in
+    a batch that one table holds. Every other token bit-identical to the calls
+    cut at the table's 1024 tokens, the routing of all of them the same."""
+    from fomoe_amd import synthetic as S
+    T, cut, bad = 1300, 1024, [0, 5, 511, 512, 1023, 1100]
+    say(f"prefill segments, non-finite tokens T={T}")
+    shape = S.LayerShape(n_embd=256, inter=256, n_experts=512, k=4, shared=True)
+    H, k = shape.n_embd, shape.k
+    L = S.build_layer(gpu, shape, 0, seed=93, zipf_s=1.1, norm=False)
+    x = gpu.download(S.tokens_bf16(gpu, T, H, seed=94), np.uint16, T * H).reshape(T, H)
+    x[bad[::2]] = 0x7FC0           # NaN rows
+    x[bad[1::2], 17] = 0x7F80      # one infinite value
+    dx, dout, d2 = gpu.upload(x), gpu.alloc(4 * T * H), gpu.alloc(4 * T * H)
+    gpu.moe_prefill(L.desc, dx, T, dout, 0)
+    got, ids = gpu.download(dout, np.uint32, T * H).reshape(T, H), gpu.prefill_routing(T, k)[0]
+    parts = []
+    for t0, n in ((0, cut), (cut, T - cut)):
+        gpu.moe_prefill(L.desc, dx.offset(2 * t0 * H), n, d2.offset(4 * t0 * H), 0)
+        parts.append(gpu.prefill_routing(n, k)[0])
+    want = gpu.download(d2, np.uint32, T * H).reshape(T, H)
+    assert np.array_equal(ids, np.concatenate(parts))
+    assert any(len(set(ids[t])) < k for t in bad)   # the case this is about
+    good = np.setdiff1d(np.arange(T), bad)
+    assert np.array_equal(got[good], want[good])
+    assert np.isfinite(got[good].view(np.float32)).all() and np.isnan(got[bad].view(np.float32)).any(1).all()
+
+
 @pytest.mark.parametrize("down", [O.Q6_K, O.Q5_K])
 def test_prefill_repeatable(gpu, down):
     """Work-groups take their items from atomic counters, so which work-group
