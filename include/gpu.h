@@ -67,7 +67,7 @@ int gpu_expert_ffn(gpu_ctx_t *ctx,
  * tiers are outside its scope), so each entry point returns the reference's
  * own "not available" result and the reference's caller takes its CPU path:
  *   gpu_register_buffers / gpu_unregister_buffers (reference gpu.h:19-22):
- *     no-ops; gpu_expert_ffn copies from pageable host memory.
+ *     no-ops; gpu_expert_ffn copies from host memory, pageable or pinned.
  *   gpu_upload_model (gpu.h:26): -1 (model.c:423 prints "GPU upload failed,
  *     CPU fallback").
  *   gpu_set_ram_cache_mb / gpu_set_vram_cache_mb (gpu.h:30, 34): recorded,

@@ -262,6 +262,49 @@ def test_expert_ffn_staged_copies(gpu, n, pad):
         assert inf_rel(out, ref) < 1e-6   # n fp32 additions of the same terms
 
 
+def test_expert_ffn_pinned_blobs(gpu):
+    """Pinned blobs are copied straight from where they lie, pageable ones of
+    the same call through the ring: bit-identical outputs whatever memory each
+    blob is in, and a call with pinned blobs only starts no ring (a context of
+    its own would hold six more threads)."""
+    import ctypes as C
+    import os
+    say("expert_ffn pinned")
+    H, F, n = 4096, 1024, 6
+    gs, ds = O.row_bytes(O.Q4_K, H) * F, O.row_bytes(O.Q6_K, F) * H
+    size = 2 * gs + ds
+    d = gpu.alloc(size * n)
+    for k, off, t, M, K in ((0, 0, O.Q4_K, F, H), (1, gs, O.Q4_K, F, H), (2, 2 * gs, O.Q6_K, H, F)):
+        gpu.synth_quant(t, 43, k, 16, 0.02, M, K, n, d.offset(off), size)
+    plain = list(gpu.download(d, np.uint8, size * n).reshape(n, size))
+    mem = C.c_void_p()              # (the HIP runtime the library is linked to)
+    gpu.lib.hipHostMalloc.argtypes, gpu.lib.hipHostFree.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint], [C.c_void_p]
+    assert gpu.lib.hipHostMalloc(C.byref(mem), n * size, 0) == 0
+    pinned = [np.ctypeslib.as_array(C.cast(mem.value + e * size, C.POINTER(C.c_uint8)), (size,)) for e in range(n)]
+    for p, b in zip(pinned, plain):
+        p[:] = b
+    h, w = O.synth_f32(44, 0, 1.0, H), np.linspace(0.3, 1.0, n).astype(np.float32)
+    own = FA.Gpu()
+    threads = lambda: len(os.listdir("/proc/self/task"))
+
+    def call(mask):
+        rc, out = own.expert_ffn(h, [pinned[e] if mask >> e & 1 else plain[e] for e in range(n)], w, H, F, gs, gs, size,
+                                 O.Q4_K, O.Q4_K, O.Q6_K)
+        assert rc == 0
+        return out
+
+    for b in (pinned[0], plain[0]):   # below a slot of the ring: the runtime's own threads exist after these
+        assert own.expert_ffn(h, [b], w, H, F, gs, gs, size, O.Q4_K, O.Q4_K, O.Q6_K)[0] == 0
+    before = threads()
+    outs = [call(0b111111)]
+    assert threads() <= before
+    outs += [call(m) for m in (0b000000, 0b000111, 0b111000, 0b100001, 0b010101)]
+    own.close()
+    gpu.lib.hipHostFree(mem)
+    for o in outs[1:]:
+        assert np.array_equal(o.view(np.uint32), outs[0].view(np.uint32))
+
+
 # ------------------------------------------------------------------ router
 @pytest.mark.parametrize("norm,bias", [(False, False), (True, True)])
 def test_router_topk(gpu, norm, bias):
