@@ -65,6 +65,7 @@ class HostStage {
         for (int u = 0; u < units; u++) done_[u].store(0, std::memory_order_relaxed);
         next_.store(0, std::memory_order_relaxed);
         limit_.store(kSlots, std::memory_order_relaxed);
+        failed_.store(false, std::memory_order_relaxed);
         hipError_t err = hipSuccess;
         // the previous run's last copies may still be on their way from the ring
         for (int k = 0; k < kSlots && err == hipSuccess; k++)
@@ -81,6 +82,7 @@ class HostStage {
             if (u >= kSlots / 2) {
                 const int old = u - kSlots / 2;
                 if (err == hipSuccess) err = hipEventSynchronize(ev_[old % kSlots]);
+                if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // the slot may still be read: it is not refilled
                 limit_.store(old + 1 + kSlots, std::memory_order_release);
             }
             const uint64_t off = (uint64_t)u * kSlot, len = total_ - off < kSlot ? total_ - off : kSlot;
@@ -135,7 +137,8 @@ class HostStage {
                 const int i = next_.fetch_add(1, std::memory_order_relaxed), u = i / kParts;
                 if (i >= n_) break;
                 while (limit_.load(std::memory_order_acquire) <= u) std::this_thread::yield();
-                part(i);
+                // (after a failure failed_ is set before the limit that lets a refill in)
+                if (u < kSlots || !failed_.load(std::memory_order_relaxed)) part(i);
                 done_[u].fetch_add(1, std::memory_order_release);
             }
             active_.fetch_sub(1, std::memory_order_release);
@@ -149,6 +152,7 @@ class HostStage {
     std::mutex m_;
     std::condition_variable cv_;
     bool quit_ = false;
+    std::atomic<bool> failed_{false};
     uint64_t job_ = 0;
     const void *const *src_ = nullptr;
     uint64_t bytes_ = 0, total_ = 0;
