@@ -588,7 +588,7 @@ static hipError_t copy_blobs(gpu_ctx *ctx, void *const *src, int n, uint64_t str
         const bool host = (uint64_t)n * stride >= HostStage::kSlot && pageable(src[e]);
         for (r = e + 1; host && r < n && pageable(src[r]);) r++;
         const uint64_t bytes = (uint64_t)(r - e) * stride;
-        const bool staged = host && bytes >= HostStage::kSlot && bytes <= HostStage::kMaxBytes;
+        const bool staged = host && bytes >= HostStage::kSlot;
         if (staged && !ctx->stage_tried) {
             ctx->stage_tried = true;
             ctx->stage = HostStage::create();
@@ -608,11 +608,14 @@ static hipError_t copy_blobs(gpu_ctx *ctx, void *const *src, int n, uint64_t str
 // Reference gpu_kernels.hip:8385-8488: same argument checks and -1 fallbacks
 // (limits MAX_EXPERTS 10, MAX_N_EMBD 4096, MAX_INTERMEDIATE 2048,
 // MAX_EXPERT_STRIDE 12 MiB at gpu_kernels.hip:438-441).
+constexpr int kFfnMaxExperts = 10;
+constexpr uint64_t kFfnMaxStride = 12ull << 20;
+static_assert(kFfnMaxExperts * kFfnMaxStride <= HostStage::kMaxBytes, "a call's blobs fit one run of the ring");
 int gpu_expert_ffn(gpu_ctx_t *ctx, const float *h, void **expert_buffers, const float *scores,
                    int n_experts, int n_embd, int inter, uint64_t gate_size, uint64_t up_size,
                    uint64_t stride, int gate_type, int up_type, int down_type, float *ffn_out) {
     if (!ctx) return -1;
-    if (n_experts > 10 || n_embd > 4096 || inter > 2048 || stride > 12ull * 1024 * 1024) return -1;
+    if (n_experts > kFfnMaxExperts || n_embd > 4096 || inter > 2048 || stride > kFfnMaxStride) return -1;
     if (!kquant(gate_type) || !kquant(up_type) || !kquant(down_type)) return -1;
     if (!h || !ffn_out || n_embd <= 0 || inter <= 0 || n_embd % 256 || inter % 256) return -1;
     if (n_experts <= 0) {

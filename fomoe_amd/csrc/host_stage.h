@@ -6,11 +6,14 @@
 // threads copy the blobs into a ring of pinned slots while the calling thread
 // hands the filled ones to the device in order: 1.81 ms for the same call with
 // slots of 8 MiB (1.95 with 4, 2.19 with 2, whatever the thread count: the
-// device's share of each copy counts). One per context (a
-// context is one host thread's), threads and slots released with it.
+// device's share of each copy counts). One per context (a context is one host
+// thread's), threads and slots released with it; the threads take no signals
+// and sleep between calls and while the ring is full.
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <pthread.h>
+#include <signal.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -26,7 +29,7 @@ class HostStage {
     static constexpr int kParts = 16;                       // parts of a slot, one device copy
     static constexpr size_t kSlot = kPart * kParts;
     static constexpr int kSlots = 4, kThreads = 6;          // one thread copies 8-10 GB/s
-    static constexpr uint64_t kMaxBytes = 256u << 20;       // of one run
+    static constexpr uint64_t kMaxBytes = 120u << 20;       // of one run: ten blobs of 12 MiB
 
     // nullptr where the threads or the pinned memory cannot be had.
     static HostStage *create() {
@@ -46,7 +49,7 @@ class HostStage {
             std::lock_guard<std::mutex> l(m_);
             quit_ = true;
         }
-        cv_.notify_all();
+        cv_.notify_all();   // (no run is under way: its caller is ours)
         for (std::thread &t : threads_) t.join();
         for (hipEvent_t e : ev_)
             if (e) (void)hipEventDestroy(e);
@@ -82,8 +85,12 @@ class HostStage {
             if (u >= kSlots / 2) {
                 const int old = u - kSlots / 2;
                 if (err == hipSuccess) err = hipEventSynchronize(ev_[old % kSlots]);
-                if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // the slot may still be read: it is not refilled
-                limit_.store(old + 1 + kSlots, std::memory_order_release);
+                {
+                    std::lock_guard<std::mutex> l(m_);
+                    if (err != hipSuccess) failed_.store(true, std::memory_order_relaxed);   // the slot may still be read: it is not refilled
+                    limit_.store(old + 1 + kSlots, std::memory_order_release);
+                }
+                room_.notify_all();
             }
             const uint64_t off = (uint64_t)u * kSlot, len = total_ - off < kSlot ? total_ - off : kSlot;
             const int parts = (int)((len + kPart - 1) / kPart), k = u % kSlots;
@@ -107,6 +114,11 @@ class HostStage {
         }
         for (hipEvent_t &e : ev_)
             if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+        struct NoSignals {   // a new thread inherits the mask: the program's handlers stay on its own threads
+            sigset_t old;
+            NoSignals() { sigset_t all; sigfillset(&all); pthread_sigmask(SIG_SETMASK, &all, &old); }
+            ~NoSignals() { pthread_sigmask(SIG_SETMASK, &old, nullptr); }
+        } no_signals;
         for (int t = 0; t < kThreads; t++) threads_.emplace_back([this] { work(); });
         return true;
     }
@@ -136,7 +148,10 @@ class HostStage {
             for (;;) {
                 const int i = next_.fetch_add(1, std::memory_order_relaxed), u = i / kParts;
                 if (i >= n_) break;
-                while (limit_.load(std::memory_order_acquire) <= u) std::this_thread::yield();
+                if (limit_.load(std::memory_order_acquire) <= u) {   // the ring is full: a device copy away
+                    std::unique_lock<std::mutex> l(m_);
+                    room_.wait(l, [&] { return limit_.load(std::memory_order_relaxed) > u; });
+                }
                 // (after a failure failed_ is set before the limit that lets a refill in)
                 if (u < kSlots || !failed_.load(std::memory_order_relaxed)) part(i);
                 done_[u].fetch_add(1, std::memory_order_release);
@@ -150,7 +165,7 @@ class HostStage {
     bool used_[kSlots] = {};
     std::vector<std::thread> threads_;
     std::mutex m_;
-    std::condition_variable cv_;
+    std::condition_variable cv_, room_;   // a new run (or the end), a slot to fill
     bool quit_ = false;
     std::atomic<bool> failed_{false};
     uint64_t job_ = 0;

@@ -61,18 +61,30 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) { the_stream()->wait(e->due)
 
 MAIN = r"""
 #include "host_stage.h"
+#include <signal.h>
 #include <stdio.h>
 #include <unistd.h>
 #define CHECK(c) do { if (!(c)) { printf("line %d: %s\n", __LINE__, #c); _exit(3); } } while (0)
+static pthread_t handled_on;
+static void on_signal(int) { handled_on = pthread_self(); }
 int main() {
     if (std::thread::hardware_concurrency() < HostStage::kThreads + 2) { puts("skipped"); return 0; }
     no_pinned() = true;
     CHECK(!HostStage::create());
     no_pinned() = false;
-    Stream s;
+    sigset_t usr1;
+    sigemptyset(&usr1);
+    sigaddset(&usr1, SIGUSR1);
+    signal(SIGUSR1, on_signal);
+    pthread_sigmask(SIG_BLOCK, &usr1, nullptr);
+    Stream s;                                        // (its thread never takes the signal)
     the_stream() = &s;
+    pthread_sigmask(SIG_UNBLOCK, &usr1, nullptr);
     HostStage *h = HostStage::create();
     CHECK(h);
+    sigset_t now;
+    pthread_sigmask(SIG_BLOCK, &usr1, &now);         // the ring's threads alone could take it from here on
+    CHECK(!sigismember(&now, SIGUSR1));              // the caller's mask is as it was
     // blobs that end inside slots and parts, more slots than the ring has, a copy that fails and
     // the run after it, the largest run
     const struct { int n; size_t bytes; int fail; } runs[] = {
@@ -94,10 +106,13 @@ int main() {
         for (auto &b : src) memset(b.data(), 0xEE, b.size());   // every source byte has been read
         s.wait(s.queued);
         if (r.fail < 0) CHECK(got == want);
+        kill(getpid(), SIGUSR1);
         printf("%d x %zu\n", r.n, r.bytes);
         fflush(stdout);
     }
     delete h;
+    pthread_sigmask(SIG_UNBLOCK, &usr1, nullptr);
+    CHECK(pthread_equal(handled_on, pthread_self()));
     puts("done");
 }
 """
