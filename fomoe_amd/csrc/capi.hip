@@ -721,6 +721,7 @@ static size_t prefill_tile_cap(int Tc, int k, int E, bool sh) {
 // Grow the workspace for passes of Tc tokens (T in all).
 static hipError_t size_prefill(gpu_ctx_t *ctx, int T, int Tc, int k, int E, int H, int F, int Fs, bool sh, bool own) {
     const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
+    const int chunk = fo::prefill_chunk_tokens(k, E, sh);
     const size_t Pact = std::max(P * F, (size_t)Tc * Fs);   // activation elements of either pass
     // xsum [Tc x H/256 x 32] fp16, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
     const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;
@@ -731,9 +732,11 @@ static hipError_t size_prefill(gpu_ctx_t *ctx, int T, int Tc, int k, int E, int 
     need(ctx->pf_w, ctx->pf_w_cap, sizeof(float) * (size_t)T * (k + 1));
     need(ctx->pf_pairpos, ctx->pf_pairpos_cap, sizeof(int32_t) * (size_t)Tc * (k + 1));
     need(ctx->pf_pairtok, ctx->pf_pairtok_cap, sizeof(int32_t) * P);
-    need(ctx->pf_tiles, ctx->pf_tiles_cap, sizeof(int32_t) * 8 * prefill_tile_cap(Tc, k, E, sh));   // tiles, then double tiles
+    // tiles, then double tiles, then thin tiles
+    need(ctx->pf_tiles, ctx->pf_tiles_cap,
+         sizeof(int32_t) * (8 * prefill_tile_cap(Tc, k, E, sh) + 4 * (size_t)fo::prefill_max_thin(Tc, k, E, sh)));
     need(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256);
-    need(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + fo::kPfSeg - 1) / fo::kPfSeg) * E);
+    need(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + chunk - 1) / chunk) * E);
     need(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact);
     if (own)   // the shared pass's output [Tc x H] (its down rows, pairs in token order)
         need(ctx->pf_ys, ctx->pf_ys_cap, sizeof(float) * (size_t)Tc * H);
@@ -793,19 +796,19 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
         return fail(ctx, -1, "moe prefill: a Q4_K shared blob and its gate size must be 16-byte aligned");
     const bool sh = L->shared != nullptr && !own;
     const int Fs = own ? L->shared_inter : F;
-    // Larger batches run as consecutive passes (the results per token are the
-    // same). A pass that the device has no memory for is halved, down to what
-    // one grouping table holds.
+    // Larger batches run as consecutive passes of whole chunks, with the same
+    // output bits however many a pass takes. A pass that the device has no
+    // memory for is halved, down to one chunk.
+    const int chunk = fo::prefill_chunk_tokens(k, E, sh);
     int Tc = fo::prefill_pass_tokens(T, k, E, sh);
-    const int t_least = std::min(T, fo::prefill_table_tokens(E));
     for (;;) {
         const hipError_t e = size_prefill(ctx, T, Tc, k, E, H, F, Fs, sh, own);
         if (e == hipSuccess) break;
-        if (e != hipErrorOutOfMemory || Tc <= t_least) HIPC(e);
+        if (e != hipErrorOutOfMemory || Tc <= chunk) HIPC(e);
         (void)hipGetLastError();
         HIPC(hipStreamSynchronize(ctx->stream));
         free_prefill(ctx);
-        Tc = std::max(t_least, Tc / 64 * 32);
+        Tc = std::max(1, (Tc + chunk - 1) / chunk / 2) * chunk;
     }
     const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
     const size_t tcap = prefill_tile_cap(Tc, k, E, sh), Pact = std::max(P * F, (size_t)Tc * Fs);
@@ -825,6 +828,7 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
     a.logits = ctx->pf_logits; a.pairpos = ctx->pf_pairpos;
     a.pair_tok = ctx->pf_pairtok; a.tiles = ctx->pf_tiles; a.n_tiles = ctx->pf_ntiles;
     a.dtiles = ctx->pf_tiles + 4 * tcap;
+    a.ttiles = ctx->pf_tiles + 8 * tcap;
     a.act_hi = ctx->pf_act; a.act_lo = ctx->pf_act + Pact; a.outp = ctx->pf_outp;
     a.xsum = (uint16_t *)ctx->pf_xsum;
     a.x16 = (uint16_t *)((uint8_t *)ctx->pf_xsum + xs_bytes);
@@ -832,6 +836,7 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
     a.pexp = a.xexp + Tc;
     a.rsplit = ctx->pf_rsplit;
     a.segs = ctx->pf_segs;
+    a.chunk = chunk;
     for (int t0 = 0; t0 < T; t0 += Tc) {
         const int n = std::min(Tc, T - t0);
         a.T = n;
@@ -840,12 +845,12 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
         a.out = d_out + (size_t)t0 * H;
         a.ids = ctx->pf_ids + (size_t)t0 * k;
         a.w = ctx->pf_w + (size_t)t0 * (k + 1);
-        if (own) {   // shared pass first: ys = shared_ffn(x) for the chunk's tokens
+        if (own) {   // shared pass first: ys = shared_ffn(x) for the pass's tokens
             fo::PrefillArgs b = a;
             b.E = 1; b.k = 1; b.F = Fs;
             b.gate_type = L->shared_gate_type; b.up_type = L->shared_up_type; b.down_type = L->shared_down_type;
             b.one_expert = 1;             // no router or combine: the down rows are ys in token order
-            b.xprep_ready = 0;            // this chunk's tokens are prepared here
+            b.xprep_ready = 0;            // this pass's tokens are prepared here
             b.router = nullptr; b.router_bias = nullptr;
             b.experts = (const uint8_t *)L->shared;
             const uint64_t sds = fomoe_row_bytes(L->shared_down_type, Fs) * (uint64_t)H;

@@ -14,7 +14,6 @@ namespace fo {
 
 constexpr int kPfMT = 64;        // tokens per GEMM tile (4 MFMA row blocks of 16)
 constexpr int kPfGroupLds = 16384;   // words of each grouping table (n_experts * ceil(tokens / 32))
-constexpr int kPfSeg = 512;          // tokens per grouping segment of a larger pass
 constexpr int kPfMaxPairs = 1 << 17; // pairs of a pass (its down outputs: 2 GiB at n_embd 4096)
 constexpr int kPfThin = 4;       // pairs of a thin tile (integer-MFMA Q6_K down path)
 constexpr int kPfGateWaves = 8;                   // gate/up work-group: 4 gate + 4 up waves (two per CU)
@@ -44,12 +43,14 @@ struct PrefillArgs {
     int32_t *pairpos;            // [T x (k+1)]: pair slot of (token, rank); rank k = shared
     int32_t *pair_tok;           // [P] token of each pair slot, grouped by expert
     int32_t *tiles;              // [max_tiles x 4] {expert (E = shared), first pair, n, order}
-    int32_t *dtiles;             // [max_tiles x 4] the same in tiles of up to 2 kPfMT pairs (k_pf_down16)
-    int32_t *n_tiles;            // [6]: tiles, tiles before the thin ones, work counter of the gate/up
-                                 // kernel, double tiles, double tiles before those of thin experts,
-                                 // the shared expert's first tile
-    int32_t *segs;               // [ceil(T / kPfSeg) x E] pairs per (segment, expert), then their first pair
+    int32_t *dtiles;             // [max_tiles x 4] the same in tiles of up to 2 kPfMT pairs, thin ones left
+                                 // out (k_pf_down16)
+    int32_t *ttiles;             // [max_thin x 4] {expert, first pair, n} of up to kPfThin thin pairs
+    int32_t *n_tiles;            // [6]: tiles, thin tiles, work counter of the gate/up kernel, double
+                                 // tiles, unused, the shared expert's first tile
+    int32_t *segs;               // [ceil(T / chunk) x E] pairs per (chunk, expert), then their first pair
                                  // slots (passes above the grouping table's size)
+    int chunk;                   // tokens per chunk (prefill_chunk_tokens of the layer; a pass starts at one)
     int max_tiles;
     uint16_t *act_hi, *act_lo;   // [P x F] SwiGLU activation as bf16 hi + lo terms (a Q6_K
                                  // down projection rewrites act_hi as fp16 rows, scale in pexp)
@@ -61,7 +62,7 @@ struct PrefillArgs {
     float *outp;                 // [P x H] fp32, per-pair down output
     int32_t *pexp;               // [P] power-of-two scale of the fp16 activation rows (Q6_K down)
     uint16_t *rsplit;            // bf16 router GEMM operands (prefill_router_ws_elems)
-    int thin_down;               // set by launch_prefill: thin tiles take k_pf_down_thin
+    int thin_down;               // set by launch_prefill: thin pairs take k_pf_down_thin
     int sh_down_type;            // -1: the shared down projection has down_type; else its own type
                                  // (gate/up and F as the routed experts), run by a launch of its own
     int down_sel;                // set by launch_prefill: 0 every expert's down projection, 1 the
@@ -91,12 +92,19 @@ inline int prefill_max_tiles(int T, int k, int E, bool shared) {
     return (prefill_pairs(T, k, shared) + kPfMT - 1) / kPfMT + E + (shared ? 1 : 0);
 }
 
-// Tokens of a pass: all that kPfMaxPairs pairs hold (weights are read once per
-// pass), and never fewer than one grouping table takes.
-inline int prefill_table_tokens(int E) { return (kPfGroupLds / E) * 32; }
+// An upper bound on the thin tiles.
+inline int prefill_max_thin(int T, int k, int E, bool shared) { return prefill_pairs(T, k, shared) / kPfThin + E + 1; }
+
+// A chunk: the tokens that one grouping table (and a pass's pairs) hold,
+// whatever the call's size. A pass is a whole number of them, as many as
+// kPfMaxPairs pairs hold (weights are read once per pass).
+inline int prefill_most_tokens(int k, bool shared) { return kPfMaxPairs / (k + (shared ? 1 : 0)) / 32 * 32; }
+inline int prefill_chunk_tokens(int k, int E, bool shared) {
+    const int table = (kPfGroupLds / E) * 32, most = prefill_most_tokens(k, shared);
+    return table < most ? table : most;
+}
 inline int prefill_pass_tokens(int T, int k, int E, bool shared) {
-    const int most = kPfMaxPairs / (k + (shared ? 1 : 0)) / 32 * 32, table = prefill_table_tokens(E);
-    const int n = most > table ? most : table;
+    const int c = prefill_chunk_tokens(k, E, shared), n = prefill_most_tokens(k, shared) / c * c;
     return T < n ? T : n;
 }
 

@@ -320,9 +320,15 @@ __global__ __launch_bounds__(256) void k_pf_topk(PrefillArgs a) {
 
 // ============================================================ P3 grouping
 // LDS: per-expert token bitmap bm[e][W] and popcount prefixes pre[e][W],
-// W = ceil(T/32) words (E * W <= kPfGroupLds, else segments of kPfSeg tokens);
-// counts and offsets over E+1 entries (entry E is the shared expert, all T
-// tokens).
+// W = ceil(T/32) words (E * W <= kPfGroupLds, else chunk by chunk); counts and
+// offsets over E+1 entries (entry E is the shared expert, all T tokens).
+//
+// Thin pairs: those of an expert with at most kPfThin pairs among the tokens of
+// a chunk (a.chunk consecutive tokens of the call). Their Q6_K down projection
+// runs on the integer path (k_pf_down_thin). A chunk is fixed by the layer's
+// shape, so which pairs are thin, and with them every output bit, does not
+// depend on how many chunks a pass takes. An expert's thin pairs follow its
+// other ones in its run of pair slots.
 // Row stride of k_pf_group's tables: W rounded up to odd
 __host__ __device__ constexpr int pf_group_stride(int W) { return W | 1; }
 
@@ -396,14 +402,13 @@ FO_DEV void pf_place(const PrefillArgs &a, const uint32_t *bm, const uint32_t *p
 }
 
 // More tokens than one work-group's tables hold (E * ceil(T / 32) words) are
-// grouped in segments of kPfSeg tokens, a work-group each: k_pf_gcount counts
-// a segment's pairs per expert, k_pf_group turns the counts into the tile
-// tables and each (segment, expert)'s first pair slot, k_pf_gplace places the
-// segment's pairs.
+// grouped by a work-group per chunk: k_pf_gcount counts a chunk's pairs per
+// expert, k_pf_group turns the counts into the tile tables and each (chunk,
+// expert)'s first pair slot, k_pf_gplace places the chunk's pairs.
 __global__ __launch_bounds__(1024) void k_pf_gcount(PrefillArgs a) {
     extern __shared__ uint32_t lds[];
-    constexpr int W = kPfSeg / 32, Ws = pf_group_stride(W);
-    const int t0 = blockIdx.x * kPfSeg, t1 = min(a.T, t0 + kPfSeg);
+    const int W = a.chunk / 32, Ws = pf_group_stride(W);
+    const int t0 = blockIdx.x * a.chunk, t1 = min(a.T, t0 + a.chunk);
     // bits, not occurrences: the ranks of a token with non-finite logits may
     // name one expert several times, and share one slot
     pf_bitmaps(a, lds, Ws, t0, t1);
@@ -417,9 +422,9 @@ __global__ __launch_bounds__(1024) void k_pf_gcount(PrefillArgs a) {
 __global__ __launch_bounds__(1024) void k_pf_gplace(PrefillArgs a) {
     extern __shared__ uint32_t lds[];
     __shared__ int s_off[1024];
-    constexpr int W = kPfSeg / 32, Ws = pf_group_stride(W);
+    const int W = a.chunk / 32, Ws = pf_group_stride(W);
     uint32_t *bm = lds, *pre = lds + a.E * Ws;
-    const int t0 = blockIdx.x * kPfSeg, t1 = min(a.T, t0 + kPfSeg);
+    const int t0 = blockIdx.x * a.chunk, t1 = min(a.T, t0 + a.chunk);
     if ((int)threadIdx.x < a.E) s_off[threadIdx.x] = a.segs[blockIdx.x * a.E + threadIdx.x];
     pf_bitmaps(a, bm, Ws, t0, t1);
     if ((int)threadIdx.x < a.E) pf_prefixes(bm, pre, Ws, W);
@@ -427,7 +432,7 @@ __global__ __launch_bounds__(1024) void k_pf_gplace(PrefillArgs a) {
     pf_place(a, bm, pre, s_off, Ws, t0, t1);
 }
 
-// n_seg: 0, or the segments k_pf_gcount counted (no bitmaps or placement here).
+// n_seg: 0, or the chunks k_pf_gcount counted (no bitmaps or placement here).
 __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     extern __shared__ uint32_t lds[];
     const int tid = threadIdx.x;
@@ -436,71 +441,77 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     uint32_t *bm = lds, *pre = lds + E * Ws;
     if (!n_seg) pf_bitmaps(a, bm, Ws, 0, a.T);
     const bool sh = a.shared != nullptr;
-    int cnt = 0;
+    int cnt = 0, thin = 0;                                                    // pairs, thin ones among them
     if (tid < E) {
         if (n_seg)
-            for (int q = 0; q < n_seg; q++) cnt += a.segs[q * E + tid];
-        else
+            for (int q = 0; q < n_seg; q++) {
+                const int c = a.segs[q * E + tid];
+                cnt += c;
+                thin += c <= kPfThin ? c : 0;
+            }
+        else {
             cnt = pf_prefixes(bm, pre, Ws, W);
+            thin = cnt <= kPfThin ? cnt : 0;
+        }
     } else if (tid == E && sh) {
         cnt = a.T;
     }
+    if (tid == E || a.one_expert) {   // every token's: the last chunk's pairs, or none
+        const int last = cnt > 0 ? cnt - (cnt - 1) / a.chunk * a.chunk : 0;
+        thin = last <= kPfThin ? last : 0;
+    }
+    // (a shared expert whose down projection runs in its own type is never thin)
+    if (!a.thin_down || (tid == E && a.sh_down_type >= 0)) thin = 0;
     // every prefix the tables need in four scans of packed fields
     constexpr int DT = 2 * kPfMT;
     const int nt = (cnt + kPfMT - 1) / kPfMT;                                 // 64-pair tiles
     // 128-pair tiles of the experts k_pf_down16 runs (dt_sel: all, routed, shared)
     const bool in_dt = a.dt_sel == 0 || tid != E;
-    const int dn = in_dt ? (cnt + DT - 1) / DT : 0;
     // The GEMMs take tiles in decreasing cost: entry i's fourth word is the
     // i-th tile by token-block count (4, 3, 2, 1; expert order within a
-    // count), so the last work handed out is the cheapest; the one tile of an
-    // expert of at most kPfThin pairs comes last of all (the thin experts,
-    // whose Q6_K down projection runs on the integer path). Per expert: its
+    // count), so the last work handed out is the cheapest. Per expert: its
     // full tiles (count 4) and its last, partial tile (count cb).
     const int nfull = cnt / kPfMT, rem = cnt - kPfMT * nfull, cb = (rem + 15) >> 4;   // cb = 0: no partial tile
-    // (a shared expert whose down projection runs in its own type is never thin)
-    const int thin = cnt > 0 && cnt <= kPfThin && !(tid == E && a.sh_down_type >= 0);
-    const int c4 = nfull + (cb == 4), c3 = cb == 3, c2 = cb == 2, c1 = cb == 1 && !thin;
-    // Double tiles for k_pf_down16: per expert ceil(cnt / 128) tiles of up to
-    // 2 kPfMT pairs (its weights are read and decoded once per 128 pairs), in
-    // decreasing token-block count (8 .. 1), those of thin experts last.
-    const int dcnt = in_dt ? cnt : 0;
+    const int c4 = nfull + (cb == 4), c3 = cb == 3, c2 = cb == 2, c1 = cb == 1;
+    // Double tiles for k_pf_down16: per expert tiles of up to 2 kPfMT of its
+    // pairs but the thin ones (its weights are read and decoded once per 128
+    // pairs), in decreasing token-block count (8 .. 1).
+    const int dcnt = in_dt ? cnt - thin : 0, dn = (dcnt + DT - 1) / DT;
     const int dfull = dcnt / DT, drem = dcnt - DT * dfull, dcb = (drem + 15) >> 4;
-    const int dthin = thin && in_dt;
-    auto cls = [&](int b) { return b == 8 ? dfull + (dcb == 8) : (dcb == b && !dthin ? 1 : 0); };
+    auto cls = [&](int b) { return b == 8 ? dfull + (dcb == 8) : (dcb == b ? 1 : 0); };
+    const int tn = (thin + kPfThin - 1) / kPfThin;                            // thin tiles
     __shared__ uint64_t scan64[4 * 16];
     const uint64_t p1 = (uint64_t)cnt | ((uint64_t)nt << 21) | ((uint64_t)dn << 42);
-    const uint64_t p2 = (uint64_t)c4 | ((uint64_t)c3 << 16) | ((uint64_t)c2 << 28) | ((uint64_t)c1 << 40) |
-                        ((uint64_t)thin << 52);
-    const uint64_t p5 = (uint64_t)dthin;   // thin experts among the double tiles
+    const uint64_t p2 = (uint64_t)c4 | ((uint64_t)c3 << 16) | ((uint64_t)c2 << 28) | ((uint64_t)c1 << 40);
     const uint64_t p3 = (uint64_t)cls(8) | ((uint64_t)cls(7) << 16) | ((uint64_t)cls(6) << 28) |
                         ((uint64_t)cls(5) << 40) | ((uint64_t)cls(4) << 52);
-    const uint64_t p4 = (uint64_t)cls(3) | ((uint64_t)cls(2) << 12) | ((uint64_t)cls(1) << 24);
+    const uint64_t p4 = (uint64_t)cls(3) | ((uint64_t)cls(2) << 12) | ((uint64_t)cls(1) << 24) | ((uint64_t)tn << 36);
     uint64_t s1, s2, s3, s4;
-    block_exclusive_scan64x4(p1, p2, p3, p4 | (p5 << 36), s1, s2, s3, s4, scan64);
+    block_exclusive_scan64x4(p1, p2, p3, p4, s1, s2, s3, s4, scan64);
     const int off = (int)fld(s1, 0, 21), toff = (int)fld(s1, 21, 21), doff = (int)fld(s1, 42, 21);
     __shared__ uint64_t s_tot[4];
-    if (tid == 1023) { s_tot[0] = s1 + p1; s_tot[1] = s2 + p2; s_tot[2] = s3 + p3; s_tot[3] = s4 + (p4 | (p5 << 36)); }
+    if (tid == 1023) { s_tot[0] = s1 + p1; s_tot[1] = s2 + p2; s_tot[2] = s3 + p3; s_tot[3] = s4 + p4; }
     if (tid == E && sh) a.n_tiles[5] = toff;   // the shared expert's first 64-pair tile
     __syncthreads();
     const uint64_t t1 = s_tot[0], t2 = s_tot[1], t3 = s_tot[2], t4 = s_tot[3];
-    const int T4 = (int)fld(t2, 0, 16), T3 = (int)fld(t2, 16, 12), T2 = (int)fld(t2, 28, 12), T1 = (int)fld(t2, 40, 12);
-    const int Tthin = (int)fld(t2, 52, 12), Tdthin = (int)fld(t4, 36, 12);
+    const int T4 = (int)fld(t2, 0, 16), T3 = (int)fld(t2, 16, 12), T2 = (int)fld(t2, 28, 12);
     const int b4 = (int)fld(s2, 0, 16);                                       // this expert's first rank per count
     const int bpart = cb == 4 ? b4 + nfull : cb == 3 ? T4 + (int)fld(s2, 16, 12)
-                    : cb == 2 ? T4 + T3 + (int)fld(s2, 28, 12) : thin ? T4 + T3 + T2 + T1 + (int)fld(s2, 52, 12)
-                    : T4 + T3 + T2 + (int)fld(s2, 40, 12);
+                    : cb == 2 ? T4 + T3 + (int)fld(s2, 28, 12) : T4 + T3 + T2 + (int)fld(s2, 40, 12);
     if (tid <= E) {
         for (int i = 0; i < nt; i++) {
             int32_t *tp = a.tiles + 4 * (toff + i);
             tp[0] = tid; tp[1] = off + kPfMT * i; tp[2] = min(kPfMT, cnt - kPfMT * i);
             a.tiles[4 * (i < nfull ? b4 + i : bpart) + 3] = toff + i;
         }
+        for (int i = 0; i < tn; i++) {
+            int32_t *tp = a.ttiles + 4 * ((int)fld(s4, 36, 21) + i);
+            tp[0] = tid; tp[1] = off + cnt - thin + kPfThin * i; tp[2] = min(kPfThin, thin - kPfThin * i);
+        }
     }
-    // [0]: tiles, [1]: tiles before the thin ones, [2]: k_pf_gateup_f16 work
-    // counter, [3]: double tiles, [4]: double tiles before the thin experts'
+    // [0]: tiles, [1]: thin tiles, [2]: k_pf_gateup_f16 work counter, [3]: double tiles
     const int NT = (int)fld(t1, 21, 21), ND = (int)fld(t1, 42, 21);
-    if (tid == 1023) { a.n_tiles[0] = NT; a.n_tiles[1] = NT - Tthin; a.n_tiles[2] = 0; a.n_tiles[3] = ND; a.n_tiles[4] = ND - Tdthin; }
+    if (tid == 1023) { a.n_tiles[0] = NT; a.n_tiles[1] = (int)fld(t4, 36, 21); a.n_tiles[2] = 0; a.n_tiles[3] = ND; }
     {
         int tot[9], base[9];   // per class count and first rank, classes in order 8, 7, .., 1
         tot[8] = (int)fld(t3, 0, 16); tot[7] = (int)fld(t3, 16, 12); tot[6] = (int)fld(t3, 28, 12);
@@ -508,16 +519,14 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
         tot[3] = (int)fld(t4, 0, 12); tot[2] = (int)fld(t4, 12, 12); tot[1] = (int)fld(t4, 24, 12);
         base[8] = 0;
         for (int b = 7; b >= 1; b--) base[b] = base[b + 1] + tot[b + 1];
-        const int thin_base = base[1] + tot[1];
         const int mine[9] = {0, (int)fld(s4, 24, 12), (int)fld(s4, 12, 12), (int)fld(s4, 0, 12), (int)fld(s3, 52, 12),
                              (int)fld(s3, 40, 12), (int)fld(s3, 28, 12), (int)fld(s3, 16, 12), (int)fld(s3, 0, 16)};
         if (tid <= E) {
             for (int i = 0; i < dn; i++) {
                 int32_t *tp = a.dtiles + 4 * (doff + i);
-                tp[0] = tid; tp[1] = off + DT * i; tp[2] = min(DT, cnt - DT * i);
+                tp[0] = tid; tp[1] = off + DT * i; tp[2] = min(DT, dcnt - DT * i);
                 int rank;
-                if (dthin) rank = thin_base + (int)fld(s4, 36, 12);
-                else if (i < dfull) rank = base[8] + mine[8] + i;
+                if (i < dfull) rank = base[8] + mine[8] + i;
                 else rank = dcb == 8 ? base[8] + mine[8] + dfull : base[dcb] + mine[dcb];
                 a.dtiles[4 * rank + 3] = doff + i;
             }
@@ -526,11 +535,12 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     // pair offsets of each expert for the placement pass
     __shared__ int s_off[1025];
     if (tid <= E) s_off[tid] = off;
-    if (n_seg && tid < E)
-        for (int q = 0, o = off; q < n_seg; q++) {
+    if (n_seg && tid < E)   // thin is 0 where the integer path is not taken
+        for (int q = 0, o = off, ot = off + cnt - thin; q < n_seg; q++) {
             const int c = a.segs[q * E + tid];
-            a.segs[q * E + tid] = o;
-            o += c;
+            int &at = thin && c <= kPfThin ? ot : o;
+            a.segs[q * E + tid] = at;
+            at += c;
         }
     __syncthreads();
     if (!n_seg) pf_place(a, bm, pre, s_off, Ws, 0, a.T);
@@ -1435,10 +1445,10 @@ __global__ __launch_bounds__(kPfD16Waves * 64, kPfD16PerCU * kPfD16Waves / 4) vo
     // (an expert's tiles are neighbours in that order; down16 HBM reads -15 %
     // against every eighth tile per XCD); its work-groups take its items
     // u = i / 8, + G8, ..., the costliest first
-    // thin experts: k_pf_down_thin; the shared expert alone: tiles of 32
+    // thin pairs: k_pf_down_thin; the shared expert alone: tiles of 32
     // pairs, so that its items (16 row blocks each) reach every work-group
     constexpr int kShTile = 32;
-    const int nt = a.d16_shared ? (a.T + kShTile - 1) / kShTile : a.n_tiles[a.thin_down ? 4 : 3];
+    const int nt = a.d16_shared ? (a.T + kShTile - 1) / kShTile : a.n_tiles[3];
     const int nrb = a.H / (32 * kPfD16Waves);
     const int x = blockIdx.x & 7, G8 = gridDim.x >> 3;
     const int nrbx = (nrb - x + 7) >> 3, n_u = nt * nrbx;     // row blocks x, x + 8, ... of every tile
@@ -1646,8 +1656,7 @@ constexpr int kPfThinUnitRows = 16 * kPfThinTPW * kPfThinWaves;    // 512 rows
 static_assert(kPfThinF == 64 * 16 && kPfThinRow == 840, "k_pf_down_thin's lane layout covers F = 1024 only");
 static_assert(kPfThin <= kPfThinWaves, "one wave prepares each pair's activation");
 
-// Whether the Q6_K down projection's thin tiles take k_pf_down_thin (the one
-// place that decides; k_pf_group orders thin tiles last whatever it says).
+// Whether the Q6_K down projection of thin pairs takes k_pf_down_thin.
 __host__ inline bool pf_thin_down(const PrefillArgs &a) {
     return a.down_type == GGML_TYPE_Q6_K && a.F == kPfThinF && a.H % kPfThinUnitRows == 0;
 }
@@ -1663,7 +1672,7 @@ __global__ __launch_bounds__(64 * kPfThinWaves) void k_pf_down_thin(PrefillArgs 
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     uint8_t *zero = sx + kPfThin * kPfThinX;
     uint8_t *tb = zero + kPfThinZero + wv * kPfThinTile;
-    const int n_thick = a.n_tiles[1], n_thin = a.n_tiles[0] - n_thick;
+    const int n_thin = a.n_tiles[1];
     // 8 tiles per wave and unit where that fills the grid twice, else 4 or 2: few thin
     // experts otherwise leave work-groups with one long unit or none (16 tokens, 49
     // thin experts: 59 -> 42 us; at 512 tokens 8 tiles stay the fastest)
@@ -1675,9 +1684,8 @@ __global__ __launch_bounds__(64 * kPfThinWaves) void k_pf_down_thin(PrefillArgs 
     const bool valid = (r >> 2) == g && L < 3;
     const uint32_t aoff = (8 * n + j) * 48 + 16 * L, soff = limb_bytes + (8 * n + j) * 8;
     for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-        const int ti = n_thick + u / upt, row0 = (u % upt) * urows + wv * 16 * tpw;
-        const int tile = a.tiles[4 * ti + 3];
-        const int4 t4 = *(const int4 *)(a.tiles + 4 * tile);
+        const int row0 = (u % upt) * urows + wv * 16 * tpw;
+        const int4 t4 = *(const int4 *)(a.ttiles + 4 * (u / upt));
         const bool shared = t4.x == a.E;
         const uint8_t *blob = shared ? a.shared : a.experts + (uint64_t)t4.x * a.stride;
         const uint64_t down_off = shared ? a.sh_gate_size + a.sh_up_size : a.gate_size + a.up_size;
@@ -1832,10 +1840,11 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
     a.down_sel = 0;
     a.d16_shared = 0;
     a.dt_sel = sep && !joint ? 1 : 0;
+    a.thin_down = rt16 && pf_thin_down(a);   // thin routed Q6_K pairs (the shared expert's where it has the type)
     const bool okt = prefill_types_ok(a.gate_type, a.up_type, a.down_type);
     const int W = (a.T + 31) / 32;
     if (!okt || a.T <= 0 || a.E <= 0 || a.E > 1023 || a.k <= 0 || a.k > a.E || a.k > kMaxK ||
-        a.H <= 0 || a.H % 256 || a.H % (32 * kPfDownWaves) || a.H % (32 * kPfD16Waves) || a.F <= 0 || a.F % 256 || a.F % kPfGateRows || (a.E * W > kPfGroupLds && (!a.segs || a.one_expert)) ||
+        a.H <= 0 || a.H % 256 || a.H % (32 * kPfDownWaves) || a.H % (32 * kPfD16Waves) || a.F <= 0 || a.F % 256 || a.F % kPfGateRows || a.chunk <= 0 || a.chunk % 32 || (a.E * W > kPfGroupLds && (!a.segs || a.one_expert || a.E * (a.chunk / 32) > kPfGroupLds)) ||
         a.max_tiles < prefill_max_tiles(a.T, a.k, a.E, a.shared != nullptr))
         return hipErrorInvalidValue;
     const bool fp16_gateup = a.gate_type == GGML_TYPE_Q4_K && a.up_type == GGML_TYPE_Q4_K;
@@ -1869,7 +1878,7 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute((const void *)k_pf_group, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            2 * (kPfGroupLds + kMaxE) * (int)sizeof(uint32_t));
         if (e != hipSuccess) return e;
-        constexpr int seg = kMaxE * pf_group_stride(kPfSeg / 32) * (int)sizeof(uint32_t);
+        constexpr int seg = (kPfGroupLds + kMaxE) * (int)sizeof(uint32_t);
         e = hipFuncSetAttribute((const void *)k_pf_gcount, hipFuncAttributeMaxDynamicSharedMemorySize, seg);
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute((const void *)k_pf_gplace, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * seg);
@@ -1879,8 +1888,8 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
     if (a.E * W <= kPfGroupLds) {
         k_pf_group<<<1, 1024, 2 * (size_t)a.E * pf_group_stride(W) * sizeof(uint32_t), s>>>(a, 0);
     } else {
-        const int n_seg = (a.T + kPfSeg - 1) / kPfSeg;
-        const size_t seg = (size_t)a.E * pf_group_stride(kPfSeg / 32) * sizeof(uint32_t);
+        const int n_seg = (a.T + a.chunk - 1) / a.chunk;
+        const size_t seg = (size_t)a.E * pf_group_stride(a.chunk / 32) * sizeof(uint32_t);
         k_pf_gcount<<<n_seg, 1024, seg, s>>>(a);
         k_pf_group<<<1, 1024, 0, s>>>(a, n_seg);
         k_pf_gplace<<<n_seg, 1024, 2 * seg, s>>>(a);
@@ -1960,7 +1969,6 @@ hipError_t launch_prefill(const PrefillArgs &a_, hipStream_t s) {
             }
             const int np = prefill_pairs(a.T, a.k, a.shared != nullptr);
             k_pf_actprep_w<<<(np + kApWaves - 1) / kApWaves, 64 * kApWaves, 0, s>>>(a, np);
-            a.thin_down = rt16 && pf_thin_down(a);   // thin routed Q6_K experts (never the shared one here)
             int dev = 0, n_cu = 256;
             if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
             const unsigned g16 = (kPfD16PerCU * n_cu + 7) & ~7;   // persistent

@@ -1448,6 +1448,50 @@ def test_prefill_pass_sizes(gpu, E, k, T, cut):
     assert np.array_equal(got, gpu.download(d2, np.uint32, T * H))
 
 
+def _own_shared(gpu, L, H, Fs, down, seed):
+    """Give layer L a shared expert of its own intermediate size; returns its device blob."""
+    parts = [O.synth_quant(O.Q4_K, seed, 0, 0.02, Fs, H), O.synth_quant(O.Q4_K, seed, 1, 0.02, Fs, H),
+             O.synth_quant(down, seed, 2, 0.02, H, Fs)]
+    blob = gpu.upload(np.concatenate(parts))
+    L.desc.shared, L.desc.shared_inter = blob.ptr, Fs
+    L.desc.shared_gate_size, L.desc.shared_up_size = parts[0].size, parts[1].size
+    L.desc.shared_gate_type, L.desc.shared_up_type, L.desc.shared_down_type = O.Q4_K, O.Q4_K, down
+    return blob
+
+
+@pytest.mark.parametrize("E,k,T,chunk,F,own", [
+    (512, 4, 2500, 1024, 1024, None),           # experts thin in some chunks and not in others
+    (512, 4, 2051, 1024, 1024, None),           # a last chunk of three tokens: the shared expert's pairs are thin there
+    (100, 4, 5218, 5216, 1024, None),           # chunks that are no power of two
+    (512, 4, 2051, 1024, 768, (1024, O.Q6_K)),  # a shared pass whose last chunk is thin, the routed pairs never
+    (512, 4, 1100, 1024, 1024, (512, O.Q8_0))])
+def test_prefill_chunks_thin(gpu, E, k, T, chunk, F, own):
+    """Which pairs of a Q6_K down projection run on the integer path is decided
+    per chunk of the call ((16384 / E) * 32 tokens), so a batch of several
+    chunks gives the bits of the calls cut at the chunks, with at most four
+    pairs of an expert in one chunk and more in another."""
+    from fomoe_amd import synthetic as S
+    say(f"prefill chunks, thin E={E} k={k} T={T} F={F} own={own}")
+    shape = S.LayerShape(n_embd=512, inter=F, n_experts=E, k=k, shared=True)
+    H = shape.n_embd
+    L = S.build_layer(gpu, shape, 0, seed=95, zipf_s=1.1, norm=False)
+    keep = _own_shared(gpu, L, H, own[0], own[1], 96) if own else None
+    dx, dout, d2 = S.tokens_bf16(gpu, T, H, seed=97), gpu.alloc(4 * T * H), gpu.alloc(4 * T * H)
+    gpu.moe_prefill(L.desc, dx, T, dout, FA.MOE_RESIDUAL)
+    got, (ids, w) = gpu.download(dout, np.uint32, T * H), gpu.prefill_routing(T, k)
+    cuts = [np.bincount(ids[t0:t0 + chunk].ravel(), minlength=E) for t0 in range(0, T, chunk)]
+    thin = [(c > 0) & (c <= 4) for c in cuts]
+    say("  thin experts per chunk:", [int(t.sum()) for t in thin])
+    if F == 1024:
+        assert any((t & (sum(cuts) > 4)).any() for t in thin)   # thin in its chunk, not in the batch
+    for t0 in range(0, T, chunk):
+        n = min(chunk, T - t0)
+        gpu.moe_prefill(L.desc, dx.offset(2 * t0 * H), n, d2.offset(4 * t0 * H), FA.MOE_RESIDUAL)
+        i2, w2 = gpu.prefill_routing(n, k)
+        assert np.array_equal(ids[t0:t0 + n], i2) and np.array_equal(w[t0:t0 + n], w2)
+    assert np.array_equal(got, gpu.download(d2, np.uint32, T * H))
+
+
 def test_prefill_segments_nonfinite_tokens(gpu):
     """Tokens with non-finite logits in a batch above one grouping table: all
     their ranks may name the same expert, whose pair then has one slot, as in
