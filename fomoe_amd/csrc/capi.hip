@@ -13,6 +13,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <array>
 #include <string>
 #include <vector>
 
@@ -21,6 +22,7 @@
 #include "kernels.h"
 #include "moe.h"
 #include "prefill.h"
+#include "prefill_ws.h"
 #include "context.h"
 
 using namespace fo;
@@ -718,50 +720,51 @@ static size_t prefill_tile_cap(int Tc, int k, int E, bool sh) {
     return (size_t)std::max(fo::prefill_max_tiles(Tc, k, E, sh), fo::prefill_max_tiles(Tc, 1, 1, false));
 }
 
-// Grow the workspace for passes of Tc tokens (T in all).
-static hipError_t size_prefill(gpu_ctx_t *ctx, int T, int Tc, int k, int E, int H, int F, int Fs, bool sh, bool own) {
+// The workspace of passes of Tc tokens (T in all).
+static std::array<fo::PfBuf, 13> prefill_bufs(gpu_ctx_t *ctx, int T, int Tc, int k, int E, int H, int F, int Fs, bool sh, bool own) {
     const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
     const int chunk = fo::prefill_chunk_tokens(k, E, sh);
     const size_t Pact = std::max(P * F, (size_t)Tc * Fs);   // activation elements of either pass
     // xsum [Tc x H/256 x 32] fp16, then x16 [Tc x H] fp16, then xexp [Tc] int32, then pexp [P] int32
     const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;
-    hipError_t e = hipSuccess;
-    auto need = [&](auto *&p, size_t &cap, size_t bytes) { if (e == hipSuccess) e = ensure(p, cap, bytes); };
-    need(ctx->pf_logits, ctx->pf_logits_cap, sizeof(float) * (size_t)Tc * E);
-    need(ctx->pf_ids, ctx->pf_ids_cap, sizeof(int32_t) * (size_t)T * k);
-    need(ctx->pf_w, ctx->pf_w_cap, sizeof(float) * (size_t)T * (k + 1));
-    need(ctx->pf_pairpos, ctx->pf_pairpos_cap, sizeof(int32_t) * (size_t)Tc * (k + 1));
-    need(ctx->pf_pairtok, ctx->pf_pairtok_cap, sizeof(int32_t) * P);
-    // tiles, then double tiles, then thin tiles
-    need(ctx->pf_tiles, ctx->pf_tiles_cap,
-         sizeof(int32_t) * (8 * prefill_tile_cap(Tc, k, E, sh) + 4 * (size_t)fo::prefill_max_thin(Tc, k, E, sh)));
-    need(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256);
-    need(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + chunk - 1) / chunk) * E);
-    need(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact);
-    if (own)   // the shared pass's output [Tc x H] (its down rows, pairs in token order)
-        need(ctx->pf_ys, ctx->pf_ys_cap, sizeof(float) * (size_t)Tc * H);
-    need(ctx->pf_outp, ctx->pf_outp_cap, sizeof(float) * P * H);
-    need(ctx->pf_rsplit, ctx->pf_rsplit_cap, sizeof(uint16_t) * fo::prefill_router_ws_elems(E, Tc, H));
-    need(ctx->pf_xsum, ctx->pf_xsum_cap, xs_bytes + x16_bytes + sizeof(int32_t) * ((size_t)Tc + P));
-    return e;
+    auto buf = [](auto *&p, size_t &cap, size_t need) { return fo::PfBuf{(void **)&p, &cap, need}; };
+    return {
+        buf(ctx->pf_logits, ctx->pf_logits_cap, sizeof(float) * (size_t)Tc * E),
+        buf(ctx->pf_ids, ctx->pf_ids_cap, sizeof(int32_t) * (size_t)T * k),
+        buf(ctx->pf_w, ctx->pf_w_cap, sizeof(float) * (size_t)T * (k + 1)),
+        buf(ctx->pf_pairpos, ctx->pf_pairpos_cap, sizeof(int32_t) * (size_t)Tc * (k + 1)),
+        buf(ctx->pf_pairtok, ctx->pf_pairtok_cap, sizeof(int32_t) * P),
+        // tiles, then double tiles, then thin tiles
+        buf(ctx->pf_tiles, ctx->pf_tiles_cap,
+            sizeof(int32_t) * (8 * prefill_tile_cap(Tc, k, E, sh) + 4 * (size_t)fo::prefill_max_thin(Tc, k, E, sh))),
+        buf(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256),
+        buf(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + chunk - 1) / chunk) * E),
+        buf(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact),
+        // the shared pass's output [Tc x H] (its down rows, pairs in token order)
+        buf(ctx->pf_ys, ctx->pf_ys_cap, own ? sizeof(float) * (size_t)Tc * H : 0),
+        buf(ctx->pf_outp, ctx->pf_outp_cap, sizeof(float) * P * H),
+        buf(ctx->pf_rsplit, ctx->pf_rsplit_cap, sizeof(uint16_t) * fo::prefill_router_ws_elems(E, Tc, H)),
+        buf(ctx->pf_xsum, ctx->pf_xsum_cap, xs_bytes + x16_bytes + sizeof(int32_t) * ((size_t)Tc + P))};
 }
 
-// Give the prefill workspace back (nothing may be running on it).
-static void free_prefill(gpu_ctx_t *ctx) {
-    auto drop = [](auto *&p, size_t &cap) {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        cap = 0;
-    };
-    drop(ctx->pf_logits, ctx->pf_logits_cap);   drop(ctx->pf_ids, ctx->pf_ids_cap);
-    drop(ctx->pf_w, ctx->pf_w_cap);             drop(ctx->pf_pairpos, ctx->pf_pairpos_cap);
-    drop(ctx->pf_pairtok, ctx->pf_pairtok_cap); drop(ctx->pf_tiles, ctx->pf_tiles_cap);
-    drop(ctx->pf_ntiles, ctx->pf_ntiles_cap);   drop(ctx->pf_segs, ctx->pf_segs_cap);
-    drop(ctx->pf_act, ctx->pf_act_cap);         drop(ctx->pf_ys, ctx->pf_ys_cap);
-    drop(ctx->pf_outp, ctx->pf_outp_cap);       drop(ctx->pf_rsplit, ctx->pf_rsplit_cap);
-    drop(ctx->pf_xsum, ctx->pf_xsum_cap);
-    ctx->pf_T = 0;                              // the last prefill's routing is gone with it
-}
+// The device as prefill_fit sees it.
+struct PrefillDev {
+    hipStream_t s;
+    hipError_t alloc(void **p, size_t bytes) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipSuccess) {
+            *p = nullptr;
+            (void)hipGetLastError();
+        }
+        return e;
+    }
+    void free(void *p) { (void)hipFree(p); }
+    hipError_t wait() { return hipStreamSynchronize(s); }
+    size_t free_bytes() {
+        size_t f = 0, all = 0;
+        return hipMemGetInfo(&f, &all) == hipSuccess ? f : 0;
+    }
+};
 
 int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_x, int n_tokens,
                     float *d_out, int flags) {
@@ -797,19 +800,13 @@ int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *L, const uint16_t *d_
     const bool sh = L->shared != nullptr && !own;
     const int Fs = own ? L->shared_inter : F;
     // Larger batches run as consecutive passes of whole chunks, with the same
-    // output bits however many a pass takes. A pass that the device has no
-    // memory for is halved, down to one chunk.
+    // output bits however many a pass takes.
     const int chunk = fo::prefill_chunk_tokens(k, E, sh);
-    int Tc = fo::prefill_pass_tokens(T, k, E, sh);
-    for (;;) {
-        const hipError_t e = size_prefill(ctx, T, Tc, k, E, H, F, Fs, sh, own);
-        if (e == hipSuccess) break;
-        if (e != hipErrorOutOfMemory || Tc <= chunk) HIPC(e);
-        (void)hipGetLastError();
-        HIPC(hipStreamSynchronize(ctx->stream));
-        free_prefill(ctx);
-        Tc = std::max(1, (Tc + chunk - 1) / chunk / 2) * chunk;
-    }
+    PrefillDev dev{ctx->stream};
+    int Tc = 0;
+    ctx->pf_T = 0;   // the last prefill's routing is overwritten, or gone with its buffer
+    const auto bufs = [&](int t) { return prefill_bufs(ctx, T, t, k, E, H, F, Fs, sh, own); };
+    HIPC(fo::prefill_fit(dev, T, fo::prefill_pass_tokens(k, E, sh), chunk, ctx->pf_refused, bufs, Tc));
     const size_t P = (size_t)fo::prefill_pairs(Tc, k, sh);
     const size_t tcap = prefill_tile_cap(Tc, k, E, sh), Pact = std::max(P * F, (size_t)Tc * Fs);
     const size_t xs_bytes = 64 * (size_t)Tc * (H / 256), x16_bytes = 2 * (size_t)Tc * H;

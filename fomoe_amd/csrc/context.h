@@ -53,6 +53,7 @@ struct gpu_ctx {
     uint16_t *pf_act = nullptr;    size_t pf_act_cap = 0;   // hi plane then lo plane
     float *pf_outp = nullptr;      size_t pf_outp_cap = 0;
     float *pf_xsum = nullptr;      size_t pf_xsum_cap = 0;
+    size_t pf_refused = SIZE_MAX;   // bytes of the smallest workspace of several chunks the device had no memory for
     uint16_t *pf_rsplit = nullptr; size_t pf_rsplit_cap = 0;   // bf16 router GEMM operands
     float *pf_ys = nullptr;        size_t pf_ys_cap = 0;       // shared-expert pass output (own types)
     int pf_T = 0, pf_k = 0;

@@ -103,9 +103,9 @@ inline int prefill_chunk_tokens(int k, int E, bool shared) {
     const int table = (kPfGroupLds / E) * 32, most = prefill_most_tokens(k, shared);
     return table < most ? table : most;
 }
-inline int prefill_pass_tokens(int T, int k, int E, bool shared) {
-    const int c = prefill_chunk_tokens(k, E, shared), n = prefill_most_tokens(k, shared) / c * c;
-    return T < n ? T : n;
+inline int prefill_pass_tokens(int k, int E, bool shared) {
+    const int c = prefill_chunk_tokens(k, E, shared);
+    return prefill_most_tokens(k, shared) / c * c;
 }
 
 // Workspace of the bf16 router GEMM (rsplit, uint16 elements): the router's

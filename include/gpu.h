@@ -304,8 +304,13 @@ void gpu_gguf_free_moe_layer(gpu_ctx_t *ctx, gpu_moe_layer_t *L);
  * as a one-expert pass whose output the routed pass adds at the shared weight;
  * n_experts <= 1023; with Q4_K gate/up, the experts and shared pointers,
  * expert_stride and the gate sizes must be multiples of 16 bytes (-1 else). A batch of more
- * than 131072 (token, expert) pairs runs as consecutive passes, and so does one that
- * the device has no workspace memory for, with the same results per token. No
+ * than 131072 (token, expert) pairs runs as consecutive passes, and so does one whose
+ * workspace would take more than half of the device's free memory, down to passes of
+ * one chunk of (16384 / n_experts) * 32 tokens (fewer where those make more than
+ * 131072 pairs). The output bits do not depend on the passes; they depend on the
+ * chunks, which start at the call's first token: with a Q6_K down projection at inter
+ * 1024 an expert with at most four pairs in a chunk runs them on exact integer weights
+ * there, any other on the fp16 ones. No
  * counterpart in the reference, which decodes prompt tokens one at a time
  * (gpu_forward). */
 int gpu_moe_prefill(gpu_ctx_t *ctx, const gpu_moe_layer_t *layer, const uint16_t *d_x, int n_tokens,
