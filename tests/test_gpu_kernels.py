@@ -1342,9 +1342,9 @@ def test_prefill_rejects_misaligned_q4k_blobs(gpu):
 
 
 def test_prefill_chunked_batch(gpu):
-    """A batch beyond the grouping table (512 experts x 1300 tokens) runs as
-    chunks of 1024 + 276 tokens: bit-identical to the two calls made
-    separately, routing of every token equal to the oracle's, and tokens on
+    """A batch beyond the grouping table (512 experts x 1300 tokens) is one
+    pass, grouped in chunks of 1024 + 276 tokens: bit-identical to the two calls
+    made separately, routing of every token equal to the oracle's, and tokens on
     both sides of the chunk boundary within the prefill bars."""
     from fomoe_amd import synthetic as S
     T, E = 1300, 512
@@ -1380,7 +1380,7 @@ def test_prefill_chunked_batch(gpu):
 def test_prefill_chunked_shared_own_types(gpu):
     """The chunked batch (512 experts x 1300 tokens: chunks of 1024 + 276)
     with the shared expert in its own types and intermediate size (Q4_K gate
-    and up, Q8_0 down, F_s = 512): the shared pass runs per chunk;
+    and up, Q8_0 down, F_s = 512): a shared pass of both chunks first;
     bit-identical to the two calls made separately, and tokens on both sides
     of the chunk boundary against the oracle with each expert's own operand
     rounding."""
@@ -1425,11 +1425,10 @@ def test_prefill_chunked_shared_own_types(gpu):
                                        (16, 4, 33000, 26208)])
 def test_prefill_pass_sizes(gpu, E, k, T, cut):
     """Passes larger than one grouping table (E * ceil(T / 32) words: counted,
-    scanned and placed in 512-token segments, the last one of 1 token, a
-    whole one, 1 of 2) and a batch above a pass's pairs (131072 with the
-    shared expert's): bit-identical to two separate calls, whose first part
-    fits one table or pass (F = 256: every expert on the same GEMM path), with
-    the same routing."""
+    scanned and placed in chunks of 1024 or, with 1023 experts, 512 tokens, the
+    last one of 1 or 512) and a batch of two passes with one table each (a
+    pass's 131072 pairs are 26208 tokens): bit-identical to two separate calls
+    (F = 256: every expert on the same GEMM path), with the same routing."""
     from fomoe_amd import synthetic as S
     say(f"prefill passes E={E} k={k} T={T}")
     shape = S.LayerShape(n_embd=256, inter=256, n_experts=E, k=k, shared=True)
@@ -1464,7 +1463,9 @@ def _own_shared(gpu, L, H, Fs, down, seed):
     (512, 4, 2051, 1024, 1024, None),           # a last chunk of three tokens: the shared expert's pairs are thin there
     (100, 4, 5218, 5216, 1024, None),           # chunks that are no power of two
     (512, 4, 2051, 1024, 768, (1024, O.Q6_K)),  # a shared pass whose last chunk is thin, the routed pairs never
-    (512, 4, 1100, 1024, 1024, (512, O.Q8_0))])
+    (512, 4, 1100, 1024, 1024, (512, O.Q8_0)),
+    (512, 16, 7169, 1024, 1024, None),             # two passes of several chunks, 4096 + 3073 tokens
+    (512, 16, 8193, 1024, 1024, (512, O.Q8_0))])   # 5120 + 3073, each behind a shared pass of its own
 def test_prefill_chunks_thin(gpu, E, k, T, chunk, F, own):
     """Which pairs of a Q6_K down projection run on the integer path is decided
     per chunk of the call ((16384 / E) * 32 tokens), so a batch of several
@@ -1490,6 +1491,37 @@ def test_prefill_chunks_thin(gpu, E, k, T, chunk, F, own):
         i2, w2 = gpu.prefill_routing(n, k)
         assert np.array_equal(ids[t0:t0 + n], i2) and np.array_equal(w[t0:t0 + n], w2)
     assert np.array_equal(got, gpu.download(d2, np.uint32, T * H))
+
+
+def test_prefill_chunks_vs_oracle(gpu):
+    """F = 1024 above the grouping table (64 experts: chunks of 8192 tokens),
+    against the oracle: experts thin in the second chunk of 108 tokens, none
+    in the whole batch. Tokens on both sides of the chunk boundary and with
+    and without thin pairs, every output."""
+    from fomoe_amd import synthetic as S
+    T, chunk = 8300, 8192
+    say(f"prefill chunks vs oracle F=1024 T={T}")
+    shape = S.LayerShape(n_embd=512, inter=1024, n_experts=64, k=4, shared=True)
+    H, k = shape.n_embd, shape.k
+    L = S.build_layer(gpu, shape, 0, seed=98, zipf_s=1.1, norm=False)
+    dx, dout = S.tokens_bf16(gpu, T, H, seed=99), gpu.alloc(4 * T * H)
+    gpu.moe_prefill(L.desc, dx, T, dout, 0)
+    got, ids = gpu.download(dout, np.float32, T * H).reshape(T, H), gpu.prefill_routing(T, k)[0]
+    x = gpu.download(dx, np.uint16, T * H).reshape(T, H)
+    d, keep = _prefill_host_layer(shape, 0, 98, True)
+    cnt = np.bincount(ids[chunk:].ravel(), minlength=shape.n_experts)
+    thin = (cnt > 0) & (cnt <= 4)
+    assert thin.any() and (np.bincount(ids.ravel(), minlength=shape.n_experts)[thin] > 4).all()
+    with_thin = chunk + np.flatnonzero(thin[ids[chunk:]].any(1))
+    without = chunk + np.flatnonzero(~thin[ids[chunk:]].any(1))
+    mask = pf_bf16_mask(shape)
+    for t in [0, 1, chunk - 1, *with_thin[:6], *without[:4], T - 1]:
+        want, oids, _ = O.moe_prefill(d, x, t, 1, 0, bf16_mask=mask)
+        exact, _, _ = O.moe_prefill(d, x, t, 1, 0, bf16_mask=mask & 3)
+        assert np.array_equal(ids[t], oids[0]), t
+        assert inf_rel(got[t], exact[0]) <= PF16_EXACT, t
+        if t not in with_thin:
+            assert inf_rel(got[t], want[0]) <= PF16_INF, t
 
 
 def test_prefill_segments_nonfinite_tokens(gpu):
