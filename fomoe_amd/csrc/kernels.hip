@@ -117,7 +117,7 @@ FO_DEV void wave_share(int64_t total, int w, int nw, int64_t &t0, int64_t &t1) {
 // y_m[r] = W_m[r,:] . x_m. Tasks are (matrix, block of P*R rows); each wave
 // takes a contiguous run of tasks and issues all loads of a task before any
 // arithmetic.
-template <int T, int U, int G, int R>
+template <int T, int U, int G, int R, bool EACH>
 __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     constexpr int P = kWave / G, ROWS = P * R;
     const int lane = threadIdx.x & 63, sub = lane / G;
@@ -132,31 +132,36 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     XRegs<T, U> X;
     int64_t cur = -1;
     // With fp32 x (xf) the work-group prepares it in LDS itself (one thread per
-    // group, bit-identical to k_xprep): the one all matrices share (xf_stride
-    // 0), or those of the at most two matrices its waves' consecutive tasks lie
+    // group, bit-identical to k_xprep): the one all matrices share or, with
+    // EACH, those of the at most two matrices its waves' consecutive tasks lie
     // in (matvec_preps_each); otherwise x comes prepared from global memory.
+    // (EACH is an instance of its own: as a branch in this one it cost launches
+    // with a shared x up to 10 %, 8192 rows of Q8_0 at K 6144 17.3 us against
+    // 15.7, and those with separate ones up to 40 %, 8 x 1024 rows of Q6_K at K
+    // 8192 30.7 against 21.7.)
     extern __shared__ __attribute__((aligned(16))) uint8_t xs_lds[];
+    constexpr int GSZ = Fmt<T>::GSZ;
     const uint8_t *xq = a.xq;
-    uint64_t xstep = a.x_stride;
+    const uint64_t xstep = EACH ? lds_round(xq_bytes(a.K, GSZ)) : a.x_stride;
     int64_t m0 = 0;
-    if (a.xf) {
-        constexpr int GSZ = Fmt<T>::GSZ;
-        const int ng = a.K / GSZ;
-        int nx = 1;
-        if (a.xf_stride) {
-            const int w0 = (int)(blockIdx.x * (blockDim.x >> 6));
-            int64_t f0, f1, l0, l1;
-            wave_share(tpm * a.n_mats, w0, nw, f0, f1);
-            wave_share(tpm * a.n_mats, w0 + (int)(blockDim.x >> 6) - 1, nw, l0, l1);
-            m0 = min(f0 / tpm, (int64_t)a.n_mats - 1);
-            nx = l1 > f0 ? (int)((l1 - 1) / tpm - m0) + 1 : 1;
-            xstep = lds_round(xq_bytes(a.K, GSZ));
-        }
+    if constexpr (EACH) {
+        const int ng = a.K / GSZ, w0 = (int)(blockIdx.x * (blockDim.x >> 6));
+        int64_t f0, f1, l0, l1;
+        wave_share(tpm * a.n_mats, w0, nw, f0, f1);
+        wave_share(tpm * a.n_mats, w0 + (int)(blockDim.x >> 6) - 1, nw, l0, l1);
+        m0 = min(f0 / tpm, (int64_t)a.n_mats - 1);
+        const int nx = l1 > f0 ? (int)((l1 - 1) / tpm - m0) + 1 : 1;
         for (int i = threadIdx.x; i < ng * nx; i += blockDim.x) {
             const int v = i / ng, g = i - v * ng;
             uint8_t *xv = xs_lds + v * xstep;
             prep_group<GSZ>(a.xf + (m0 + v) * a.xf_stride + g * GSZ, xv + g * (kLimbs * GSZ), xv + xq_limb_bytes(a.K) + g * 8);
         }
+        __syncthreads();
+        xq = xs_lds;
+    } else if (a.xf) {
+        const int ng = a.K / GSZ;
+        for (int g = threadIdx.x; g < ng; g += blockDim.x)
+            prep_group<GSZ>(a.xf + g * GSZ, xs_lds + g * (kLimbs * GSZ), xs_lds + xq_limb_bytes(a.K) + g * 8);
         __syncthreads();
         xq = xs_lds;
     }
@@ -174,7 +179,7 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     for (int64_t t = t0; t < t1; t++) {
         const int64_t m = t / tpm;
         const int rb = (int)(t - m * tpm);
-        if (m != cur && (cur < 0 || xstep)) X.load(L, xq + (m - m0) * xstep, a.K);
+        if (m != cur && (cur < 0 || xstep)) X.load(L, xq + (EACH ? m - m0 : m) * xstep, a.K);
         cur = m;
         const uint8_t *W = a.W + m * a.mat_stride;
         RowRaw<T, U> raw[R];
@@ -231,9 +236,14 @@ static hipError_t matvec_t(const MatvecArgs &a, hipStream_t s, int n_cu) {
     const int P = 64 / G;
     const int64_t tasks = (int64_t)((a.M + P * R - 1) / (P * R)) * a.n_mats;
     const int blocks = (waves_for(tasks, n_cu, 16) + 3) / 4;
-    const size_t lds = a.xf ? lds_round(xq_bytes(a.K, Fmt<T>::GSZ)) * (a.xf_stride ? 2 : 1) : 0;
+    const bool each = a.xf && a.xf_stride;
+    const size_t lds = a.xf ? lds_round(xq_bytes(a.K, Fmt<T>::GSZ)) * (each ? 2 : 1) : 0;
 #define FO_MV(GG, UU) \
-    if (G == GG && U == UU) { k_matvec<T, UU, GG, R><<<blocks, 256, lds, s>>>(a); return hipGetLastError(); }
+    if (G == GG && U == UU) { \
+        if (each) k_matvec<T, UU, GG, R, true><<<blocks, 256, lds, s>>>(a); \
+        else k_matvec<T, UU, GG, R, false><<<blocks, 256, lds, s>>>(a); \
+        return hipGetLastError(); \
+    }
     FO_MV(64, 1) FO_MV(64, 2) FO_MV(64, 3) FO_MV(64, 4)
     FO_MV(32, 1) FO_MV(16, 1) FO_MV(8, 1) FO_MV(4, 1)
 #undef FO_MV

@@ -220,7 +220,8 @@ def test_matvec_batched(gpu, t, M, K, per_x):
     # separate x on the general kernel: work-groups inside one matrix, across two (odd
     # task counts), and matrices too small for that (prepared by a launch of their own)
     (O.Q5_K, 1000, 2816, 3, True), (O.Q5_K, 37, 2816, 7, True), (O.Q6_K, 61, 2048, 50, True),
-    (O.Q8_0, 33, 96, 40, True), (O.Q4_K, 1, 512, 3, True), (O.Q6_K, 9, 16384, 2, True)])
+    (O.Q8_0, 33, 96, 40, True), (O.Q4_K, 1, 512, 3, True), (O.Q6_K, 9, 16384, 2, True), (O.Q6_K, 1021, 8192, 5, True),
+    (O.Q8_0, 515, 8192, 9, True)])
 def test_matvec_general_routes(gpu, t, M, K, n, per_x):
     say("matvec routes", t, M, K, n, per_x)
     stride = O.row_bytes(t, K) * M
