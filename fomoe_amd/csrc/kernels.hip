@@ -804,9 +804,20 @@ static bool tile_shape(int type, uint64_t row_bytes, int K) {
 // 4096 5.1 / 6.3 / 8.5 against 7.8 / 8.2 / 8.7; Q6_K K 1024 4.6 / 4.8 / 5.4
 // against 8.6 / 8.9 / 9.0; Q8_0 K 4096 5.8 / 8.8 / 13.6 against 15.0 / 15.3 /
 // 15.8. The two meet between 18 MB (Q8_0, K 1024) and 75 MB (Q4_K, K 8192).
+// Matrices of so few rows that a tile kernel's wave has no chain of tiles stay
+// with it, where it has 16-row tiles (K <= 1024) or is Q8_0's of four (4.8
+// against 5.8 for 64 of four rows at K 4096; the other types' take longer than
+// the general kernel at any size): 512 of 16 rows 4.4 / 5.0 / 5.5
+// against 5.6 / 5.5 / 5.7 (Q6_K K 512 / 768 / 1024), 5.4 against 5.8 (Q5_K), 5.7
+// against 6.3 (Q8_0); 32 rows of K 512 5.0 against 5.8, of K 768 (20 KB) 5.3
+// against 4.9. Rows of one super-block do at any size: 1.6 MB 4.4 against 5.3,
+// 13 MB 6.5 against 7.2.
 constexpr uint64_t kSmallBytes = 16u << 20;
-static bool small_launch(const MatvecArgs &a) {
-    return a.xf && (a.xf_stride == 0 || a.n_mats == 1) && (uint64_t)a.M * a.n_mats * a.row_bytes < kSmallBytes;
+constexpr uint64_t kTileWaveBytes = 18u << 10;   // one 16-row tile of Q8_0 at K = 1024: 17 KiB
+static bool small_launch(int type, const MatvecArgs &a) {
+    if (!a.xf || a.xf_stride || (uint64_t)a.M * a.n_mats * a.row_bytes >= kSmallBytes) return false;
+    const int rows = a.K <= 1024 ? 16 : type == GGML_TYPE_Q8_0 ? 4 : 0;   // of a tile
+    return !rows || (a.K > 256 && (uint64_t)((a.M + rows - 1) / rows * rows) * a.row_bytes > kTileWaveBytes);
 }
 
 // Whether the general kernel prepares the separate x of every matrix itself: a
@@ -829,17 +840,17 @@ bool matvec_self_prep(int type, uint64_t row_bytes, int K, uint64_t x_stride) {
                              type == GGML_TYPE_Q8_0 || type == GGML_TYPE_MXFP4);
 }
 
-hipError_t launch_matvec(int type, const MatvecArgs &a, hipStream_t s, int n_cu) {
+hipError_t launch_matvec(int type, const MatvecArgs &a_, hipStream_t s, int n_cu) {
+    MatvecArgs a = a_;
     if (a.M <= 0 || a.n_mats <= 0) return hipErrorInvalidValue;
-    if (small_launch(a) && geometry_ok(type, a.K)) {
-        MatvecArgs b = a;
-        b.xf_stride = 0;   // one x
+    if (a.n_mats == 1) a.xf_stride = 0;   // one x
+    if (small_launch(type, a) && geometry_ok(type, a.K)) {
         switch (type) {
-            case GGML_TYPE_Q4_K: return matvec_t<GGML_TYPE_Q4_K, 2>(b, s, n_cu);
-            case GGML_TYPE_Q5_K: return matvec_t<GGML_TYPE_Q5_K, 2>(b, s, n_cu);
-            case GGML_TYPE_Q6_K: return matvec_t<GGML_TYPE_Q6_K, 2>(b, s, n_cu);
-            case GGML_TYPE_Q8_0: return matvec_t<GGML_TYPE_Q8_0, 2>(b, s, n_cu);
-            case GGML_TYPE_MXFP4: return matvec_t<GGML_TYPE_MXFP4, 2>(b, s, n_cu);
+            case GGML_TYPE_Q4_K: return matvec_t<GGML_TYPE_Q4_K, 2>(a, s, n_cu);
+            case GGML_TYPE_Q5_K: return matvec_t<GGML_TYPE_Q5_K, 2>(a, s, n_cu);
+            case GGML_TYPE_Q6_K: return matvec_t<GGML_TYPE_Q6_K, 2>(a, s, n_cu);
+            case GGML_TYPE_Q8_0: return matvec_t<GGML_TYPE_Q8_0, 2>(a, s, n_cu);
+            case GGML_TYPE_MXFP4: return matvec_t<GGML_TYPE_MXFP4, 2>(a, s, n_cu);
             default: return hipErrorInvalidValue;
         }
     }

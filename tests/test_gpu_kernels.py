@@ -217,6 +217,10 @@ def test_matvec_batched(gpu, t, M, K, per_x):
     # either side of the 16 MiB below which a launch with one x runs on the general kernel
     (O.Q4_K, 1024, 4096, 7, False), (O.Q4_K, 1024, 4096, 8, False), (O.Q6_K, 4096, 1024, 4, False),
     (O.Q6_K, 4096, 1024, 5, False), (O.Q8_0, 17, 1024, 1, True),
+    # and of the rows that a tile kernel's wave takes in one tile or few
+    (O.Q6_K, 16, 1024, 40, False), (O.Q6_K, 17, 1024, 40, False), (O.Q6_K, 32, 512, 33, False),
+    (O.Q6_K, 33, 512, 33, False), (O.Q6_K, 130, 256, 9, False), (O.Q5_K, 16, 1024, 33, False),
+    (O.Q5_K, 17, 1024, 33, False), (O.Q8_0, 4, 4096, 33, False), (O.Q8_0, 5, 4096, 33, False), (O.Q8_0, 1, 4096, 1, True),
     # separate x on the general kernel: work-groups inside one matrix, across two (odd
     # task counts), and matrices too small for that (prepared by a launch of their own)
     (O.Q5_K, 1000, 2816, 3, True), (O.Q5_K, 37, 2816, 7, True), (O.Q6_K, 61, 2048, 50, True),
