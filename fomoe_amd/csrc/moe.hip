@@ -406,9 +406,10 @@ hipError_t launch_expand(int type, const ExpandArgs &a, hipStream_t s, int n_cu)
     const int n_tot = a.k + (a.shared ? 1 : 0);
     const size_t lds = lds_round(xq_bytes(a.H, type == GGML_TYPE_Q6_K ? 16 : 32));
     const int grid = a.F / TR * n_tot;
-    // gate/up at H = 4096: row spans through LDS, 16 rows per work-group; a
-    // down projection with groups of 32 takes the fp32 activations instead
-    if (type == GGML_TYPE_Q4_K && (TR == 16 || (a.act_only && a.act)) && G == 64 && U == 1) {
+    // gate/up at H = 4096: row spans through LDS, 16 rows per work-group (its
+    // row bytes are that H's: no other one may come here); a down projection
+    // with groups of 32 takes the fp32 activations instead
+    if (type == GGML_TYPE_Q4_K && (TR == 16 || (a.act_only && a.act)) && a.H == 4096) {
         k_expand_q4t<<<a.F / 16 * n_tot, 256, lds + 512 + 4 * 16 * 576, s>>>(a);
         return hipGetLastError();
     }

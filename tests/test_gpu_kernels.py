@@ -425,6 +425,57 @@ def test_moe_layer_small_grids(gpu, H, F, E, k):
     assert inf_rel(got, want) < 1e-5
 
 
+@pytest.mark.parametrize("H,F,shared,gate,down", [
+    (3072, 512, False, O.Q4_K, O.Q6_K), (3072, 1024, True, O.Q4_K, O.Q6_K), (3072, 768, True, O.Q4_K, O.Q8_0),
+    (3072, 1024, True, O.Q4_K, O.Q5_K), (3072, 1024, True, O.Q5_K, O.Q6_K), (1536, 1024, True, O.Q4_K, O.Q6_K)])
+def test_moe_layer_widths(gpu, H, F, shared, gate, down):
+    """Widths whose rows fill neither 32 nor 64 slots of a wave: at 3072 Q4_K
+    gate/up took the kernel whose row bytes are those of 4096. Every expert's
+    blob is followed by bytes that decode to NaN, so a row read past it shows.
+    Outputs against the fp32 oracle."""
+    say(f"layer width H={H} F={F} shared={shared} gate={gate} down={down}")
+    E, k = 8, 3
+    gs, ds = F * O.row_bytes(gate, H), H * O.row_bytes(down, F)
+    size = 2 * gs + ds
+    stride = (size + 16 * O.row_bytes(gate, H) + 15) // 16 * 16
+    blobs = np.full(((E + shared) * stride), 0xFF, np.uint8)
+    for e in range(E + shared):
+        parts = [O.synth_quant(gate, 75, 8 * e, 0.02, F, H), O.synth_quant(gate, 75, 8 * e + 1, 0.02, F, H),
+                 O.synth_quant(down, 75, 8 * e + 2, 0.02, H, F)]
+        blobs[e * stride:e * stride + size] = np.concatenate(parts)
+    router, h = O.synth_f32(76, 0, 0.02, E * H), O.synth_f32(76, 1, 1.0, H)
+    norm = O.synth_f32(76, 2, 1.0, H)
+    keep = [gpu.upload(blobs), gpu.upload(router), gpu.upload(norm)]
+    dh, dout = gpu.upload(h), gpu.alloc(4 * H)
+
+    def fill(d, experts, r, norm_w):
+        d.n_embd, d.inter, d.n_experts, d.k = H, F, E, k
+        d.gate_type = d.up_type = gate
+        d.down_type, d.gate_size, d.up_size, d.expert_stride = down, gs, gs, stride
+        d.router, d.experts, d.norm_w, d.eps = r, experts, norm_w, 1e-6
+        if shared:
+            d.shared, d.shared_inter, d.shared_gate_size, d.shared_up_size = experts + E * stride, F, gs, gs
+            d.shared_gate_type = d.shared_up_type = gate
+            d.shared_down_type = down
+        return d
+
+    L = fill(FA.MoeLayer(), *(b.ptr for b in keep))
+    host = fill(O.MoeDesc(), blobs.ctypes.data, router.ctypes.data, norm.ctypes.data)
+    gpu.moe_layer(L, dh, dout, 0)
+    got = gpu.download(dout, np.float32, H)
+    ids, w, _ = gpu.last_routing(k)
+    want, oi, ow = O.moe_layer(host, h, 0)
+    assert np.array_equal(ids, oi)
+    assert inf_rel(w, ow) < 1e-5
+    assert inf_rel(got, want) < 1e-5
+    dx = gpu.upload(h)
+    gpu.stack_decode([L, L], dx, 1)
+    x = h
+    for _ in range(2):
+        x = O.moe_layer(host, x, O.MOE_NORM | O.MOE_RESIDUAL)[0]
+    assert inf_rel(gpu.download(dx, np.float32, H), x) < 1e-5
+
+
 @pytest.mark.parametrize("E,H", [(1, 512), (15, 1024), (16, 512), (1023, 8192)])
 def test_route_gate_vector(gpu, E, H):
     """The shared-expert gate as the router kernel's work-group of its own,
