@@ -646,11 +646,17 @@ hipError_t launch_reduce(int type, const ReduceArgs &a, hipStream_t s, int n_cu)
         if (type == GGML_TYPE_Q5_K) return reduce_tile<GGML_TYPE_Q5_K, 16, 704>(a, s);
     }
     if (a.act_f32) return hipErrorInvalidValue;   // only the LDS-staged kernel prepares from fp32
-    // passes of 64 / G rows per wave: fewer where four of them leave CUs without
-    // a work-group (H = 2048, F = 768, 8 experts:
-    // 5.7 us with two passes and 256 work-groups, 7.7 with four, 7.3 with one)
+    // Passes of 64 / G rows per wave: fewer where they leave CUs without a
+    // work-group, as long as the work-groups stay one round of the CUs, or two for
+    // a few experts, whose work-groups of few waves share a CU. A layer of a
+    // replayed stack, us with four / two / one (work-groups 192 / 384 / 768: H 1536,
+    // F 1536, Q4_K): 16 experts 30.5 / 38.3 / 37.0, 8 20.5 / 22.1 / 22.1, one 14.5 /
+    // 14.6 / 14.0; 128 / 256 / 512 (H 2048, F 768, Q6_K): 27.8 / 24.7 / 27.5, 19.8 /
+    // 18.2 / 19.3, 13.8 / 13.4 / 13.5; 64 and less: one pass, up to 4.4 under four.
+    // Over 966 shapes within about 2 % of four passes or below.
     int RP = 4;
-    while (RP > 1 && (a.H + 64 / G * RP - 1) / (64 / G * RP) < n_cu) RP >>= 1;
+    auto groups = [&](int passes) { return (a.H + 64 / G * passes - 1) / (64 / G * passes); };
+    while (RP > 1 && groups(RP) < n_cu && groups(RP / 2) <= n_cu * (n_tot <= 4 ? 2 : 1)) RP >>= 1;
     const int RB = (64 / G) * RP;
     const int grid = (a.H + RB - 1) / RB;
     const int threads = 64 * n_tot;

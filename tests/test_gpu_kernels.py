@@ -403,7 +403,8 @@ def test_moe_layer_norm_residual_gate(gpu):
 
 
 @pytest.mark.parametrize("H,F,E,k", [(4096, 768, 16, 3), (2048, 768, 128, 8), (1024, 768, 129, 8), (512, 256, 128, 16),
-                                     (1536, 1280, 127, 2)])
+                                     (1536, 1280, 127, 2), (1536, 1280, 16, 6), (3072, 512, 16, 9), (3072, 512, 16, 8),
+                                     (1536, 2048, 16, 16)])
 def test_moe_layer_small_grids(gpu, H, F, E, k):
     """The general down kernel with four, two and one passes per wave (its
     grid against the CU count; 1280: more lanes per row, fewer rows), and the
