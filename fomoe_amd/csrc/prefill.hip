@@ -469,23 +469,32 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     const bool in_dt = a.dt_sel == 0 || tid != E;
     // The GEMMs take tiles in decreasing cost: entry i's fourth word is the
     // i-th tile by token-block count (4, 3, 2, 1; expert order within a
-    // count), so the last work handed out is the cheapest. Per expert: its
+    // count), so the last work handed out is the cheapest; the one tile of an
+    // expert of at most kPfThin pairs comes last of all. Per expert: its
     // full tiles (count 4) and its last, partial tile (count cb).
     const int nfull = cnt / kPfMT, rem = cnt - kPfMT * nfull, cb = (rem + 15) >> 4;   // cb = 0: no partial tile
-    const int c4 = nfull + (cb == 4), c3 = cb == 3, c2 = cb == 2, c1 = cb == 1;
+    const bool sep_sh = tid == E && a.sh_down_type >= 0;                     // (not the shared expert of an own down type)
+    const int few = cnt > 0 && cnt <= kPfThin && !sep_sh;
+    const int c4 = nfull + (cb == 4), c3 = cb == 3, c2 = cb == 2, c1 = cb == 1 && !few;
     // Double tiles for k_pf_down16: per expert tiles of up to 2 kPfMT of its
     // pairs but the thin ones (its weights are read and decoded once per 128
-    // pairs), in decreasing token-block count (8 .. 1).
+    // pairs), in decreasing token-block count (8 .. 1), those of at most kPfThin
+    // pairs last (300 experts, 137 tokens, where the integer path is not taken:
+    // k_pf_down16 46.6 us against 52.4 with them in expert order).
     const int dcnt = in_dt ? cnt - thin : 0, dn = (dcnt + DT - 1) / DT;
     const int dfull = dcnt / DT, drem = dcnt - DT * dfull, dcb = (drem + 15) >> 4;
-    auto cls = [&](int b) { return b == 8 ? dfull + (dcb == 8) : (dcb == b ? 1 : 0); };
+    const int dfew = dcnt > 0 && dcnt <= kPfThin && !sep_sh;
+    auto cls = [&](int b) { return b == 8 ? dfull + (dcb == 8) : (dcb == b && !dfew ? 1 : 0); };
     const int tn = (thin + kPfThin - 1) / kPfThin;                            // thin tiles
+    static_assert(kPfMaxPairs / kPfThin + 1025 < 1 << 16, "thin tiles take 16 bits");
     __shared__ uint64_t scan64[4 * 16];
     const uint64_t p1 = (uint64_t)cnt | ((uint64_t)nt << 21) | ((uint64_t)dn << 42);
-    const uint64_t p2 = (uint64_t)c4 | ((uint64_t)c3 << 16) | ((uint64_t)c2 << 28) | ((uint64_t)c1 << 40);
+    const uint64_t p2 = (uint64_t)c4 | ((uint64_t)c3 << 16) | ((uint64_t)c2 << 28) | ((uint64_t)c1 << 40) |
+                        ((uint64_t)few << 52);
     const uint64_t p3 = (uint64_t)cls(8) | ((uint64_t)cls(7) << 16) | ((uint64_t)cls(6) << 28) |
                         ((uint64_t)cls(5) << 40) | ((uint64_t)cls(4) << 52);
-    const uint64_t p4 = (uint64_t)cls(3) | ((uint64_t)cls(2) << 12) | ((uint64_t)cls(1) << 24) | ((uint64_t)tn << 36);
+    const uint64_t p4 = (uint64_t)cls(3) | ((uint64_t)cls(2) << 12) | ((uint64_t)cls(1) << 24) | ((uint64_t)tn << 36) |
+                        ((uint64_t)dfew << 52);
     uint64_t s1, s2, s3, s4;
     block_exclusive_scan64x4(p1, p2, p3, p4, s1, s2, s3, s4, scan64);
     const int off = (int)fld(s1, 0, 21), toff = (int)fld(s1, 21, 21), doff = (int)fld(s1, 42, 21);
@@ -494,10 +503,11 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
     if (tid == E && sh) a.n_tiles[5] = toff;   // the shared expert's first 64-pair tile
     __syncthreads();
     const uint64_t t1 = s_tot[0], t2 = s_tot[1], t3 = s_tot[2], t4 = s_tot[3];
-    const int T4 = (int)fld(t2, 0, 16), T3 = (int)fld(t2, 16, 12), T2 = (int)fld(t2, 28, 12);
+    const int T4 = (int)fld(t2, 0, 16), T3 = (int)fld(t2, 16, 12), T2 = (int)fld(t2, 28, 12), T1 = (int)fld(t2, 40, 12);
     const int b4 = (int)fld(s2, 0, 16);                                       // this expert's first rank per count
     const int bpart = cb == 4 ? b4 + nfull : cb == 3 ? T4 + (int)fld(s2, 16, 12)
-                    : cb == 2 ? T4 + T3 + (int)fld(s2, 28, 12) : T4 + T3 + T2 + (int)fld(s2, 40, 12);
+                    : cb == 2 ? T4 + T3 + (int)fld(s2, 28, 12) : few ? T4 + T3 + T2 + T1 + (int)fld(s2, 52, 12)
+                    : T4 + T3 + T2 + (int)fld(s2, 40, 12);
     if (tid <= E) {
         for (int i = 0; i < nt; i++) {
             int32_t *tp = a.tiles + 4 * (toff + i);
@@ -505,13 +515,13 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
             a.tiles[4 * (i < nfull ? b4 + i : bpart) + 3] = toff + i;
         }
         for (int i = 0; i < tn; i++) {
-            int32_t *tp = a.ttiles + 4 * ((int)fld(s4, 36, 21) + i);
+            int32_t *tp = a.ttiles + 4 * ((int)fld(s4, 36, 16) + i);
             tp[0] = tid; tp[1] = off + cnt - thin + kPfThin * i; tp[2] = min(kPfThin, thin - kPfThin * i);
         }
     }
     // [0]: tiles, [1]: thin tiles, [2]: k_pf_gateup_f16 work counter, [3]: double tiles
     const int NT = (int)fld(t1, 21, 21), ND = (int)fld(t1, 42, 21);
-    if (tid == 1023) { a.n_tiles[0] = NT; a.n_tiles[1] = (int)fld(t4, 36, 21); a.n_tiles[2] = 0; a.n_tiles[3] = ND; }
+    if (tid == 1023) { a.n_tiles[0] = NT; a.n_tiles[1] = (int)fld(t4, 36, 16); a.n_tiles[2] = 0; a.n_tiles[3] = ND; }
     {
         int tot[9], base[9];   // per class count and first rank, classes in order 8, 7, .., 1
         tot[8] = (int)fld(t3, 0, 16); tot[7] = (int)fld(t3, 16, 12); tot[6] = (int)fld(t3, 28, 12);
@@ -526,7 +536,8 @@ __global__ __launch_bounds__(1024) void k_pf_group(PrefillArgs a, int n_seg) {
                 int32_t *tp = a.dtiles + 4 * (doff + i);
                 tp[0] = tid; tp[1] = off + DT * i; tp[2] = min(DT, dcnt - DT * i);
                 int rank;
-                if (i < dfull) rank = base[8] + mine[8] + i;
+                if (dfew) rank = base[1] + tot[1] + (int)fld(s4, 52, 12);
+                else if (i < dfull) rank = base[8] + mine[8] + i;
                 else rank = dcb == 8 ? base[8] + mine[8] + dfull : base[dcb] + mine[dcb];
                 a.dtiles[4 * rank + 3] = doff + i;
             }
