@@ -906,16 +906,15 @@ __global__ __launch_bounds__(kPfGateWaves * 64, 4) void k_pf_gateup(PrefillArgs 
 // A Q4_K weight is d * sc_j * q - dmin * m_j (q 4-bit, sc_j / m_j 6-bit
 // per 32-value sub-block j, d / dmin fp16 per super-block). sc_j * q <= 945
 // is an exact fp16 integer, so the B operand of v_mfma_f32_16x16x32_f16 is
-// built as fp16(sc_j * q) (v_perm of the code bytes under 0x64 gives
-// 1024 + q, one v_pk_fma_f16 (1024 + q) * sc - 1024 * sc gives sc * q
-// exactly) and the MFMA accumulates a whole super-block: per output
-// acc += d * D with D = sum_k x_k sc_j q_k, one fma per super-block instead
-// of one scale per 32 values. The min term -sum_j (dmin m_j) S_j (S_j the
-// token's sub-block sums, fp32) runs on v_mfma_f32_16x16x4_f32 into the same
-// accumulator. The token rows (and their sums) enter scaled by a per-token
-// power of two (k_pf_xprep: the row maximum lands in [2^14, 2^15), so the
-// fp16 rows are exact for every value above 2^-28 of the row maximum and off
-// by at most 2^-39 of it below), which the epilogue undoes.
+// sc_j * q * 2^-14 (q4_codes_f16) and the MFMA accumulates a whole super-block:
+// per output acc += d * 2^14 * D with D = sum_k x_k sc_j q_k * 2^-14, one fma per
+// super-block instead of one scale per 32 values. The min term -sum_j (dmin
+// m_j) S_j (S_j the token's sub-block sums as three fp16 terms, pf_put_sum) is one
+// more fp16 MFMA of its own accumulator, which enters the output by an fma with
+// dmin. The token rows (and their sums) enter scaled by a per-token power of two
+// (k_pf_xprep: the row maximum lands in [2^14, 2^15), so the fp16 rows are exact
+// for every value above 2^-28 of the row maximum and off by at most 2^-39 of it
+// below), which the epilogue undoes.
 //
 // Work item = (tile, 128 rows of F); work-group = 4 waves, wave w owns 32 gate
 // rows and the same 32 up rows of the item, as four blocks of 16 that share
@@ -1100,32 +1099,33 @@ constexpr uint32_t kGuA = kPfMT * 512;                // 32 KiB of token rows
 constexpr uint32_t kGuS = kPfMT * 64;                 // 4 KiB: their sub-block sums (fp16 terms)
 constexpr uint32_t kGuW = 4 * kGuHalf;                // a wave's weights: 32 gate and 32 up rows
 constexpr int kGuWaves = 4;
+constexpr int kGuBlocks = 4;                          // 16-row blocks of a wave: two of gate, two of up
 constexpr uint32_t kGuLds = kGuA + kGuS + kGuWaves * kGuW;   // 72 KiB: two work-groups per CU
 
-// One super-block of NM blocks of 16 weight rows (row col of block g at rw +
+// One super-block of kGuBlocks blocks of 16 weight rows (row col of block g at rw +
 // g * gstride, 144 bytes of it) times NB blocks of 16 tokens: token operand
 // (c, h) of block tb at ab + aoff[c] + 256 h + 8192 tb, its sums at sb + 1024
 // tb. Lane group kg owns sub-blocks 2 kg and 2 kg + 1 (MFMA (c, h): its eight
 // values are values 8c..8c+7 of sub-block 2 kg + h in pf_x16_src order), so a
-// lane decodes two scales instead of eight; the NM blocks share every token
+// lane decodes two scales instead of eight; the blocks share every token
 // operand read. Each (row, token) sees the same operations in the same order
-// whatever NM and NB.
-template <int NM, int NB>
-FO_DEV void q4_super_block(f32x4 (&acc)[NM][NB], const uint8_t *rw, uint32_t gstride, const uint8_t *ab,
+// whatever NB.
+template <int NB>
+FO_DEV void q4_super_block(f32x4 (&acc)[kGuBlocks][NB], const uint8_t *rw, uint32_t gstride, const uint8_t *ab,
                            const uint32_t (&aoff)[4], const uint8_t *sb, int col, int kg) {
-    f16x2 sp[NM][2];
-    f32x4 dd[NM][NB];
+    f16x2 sp[kGuBlocks][2];
+    f32x4 dd[kGuBlocks][NB];
 #pragma unroll
-    for (int g = 0; g < NM; g++) {
+    for (int g = 0; g < kGuBlocks; g++) {
         q4_scale_pair(*(const uint4 *)(rw + g * gstride), kg, sp[g]);
 #pragma unroll
         for (int tb = 0; tb < NB; tb++) dd[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        f16x8 bw[NM][2];
+        f16x8 bw[kGuBlocks][2];
 #pragma unroll
-        for (int g = 0; g < NM; g++)
+        for (int g = 0; g < kGuBlocks; g++)
             q4_codes_f16(*(const uint2 *)(rw + g * gstride + 16 + 32 * kg + 8 * c), sp[g], bw[g][0], bw[g][1]);
 #pragma unroll
         for (int h = 0; h < 2; h++)
@@ -1133,15 +1133,15 @@ FO_DEV void q4_super_block(f32x4 (&acc)[NM][NB], const uint8_t *rw, uint32_t gst
             for (int tb = 0; tb < NB; tb++) {
                 const f16x8 av = *(const f16x8 *)(ab + aoff[c] + 256 * h + 8192 * tb);
 #pragma unroll
-                for (int g = 0; g < NM; g++)
+                for (int g = 0; g < kGuBlocks; g++)
                     dd[g][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw[g][h], dd[g][tb], 0, 0, 0);
             }
-        if constexpr (NM * NB > 8) __builtin_amdgcn_sched_barrier(0);   // keeps the live operands few
+        if constexpr (NB > 2) __builtin_amdgcn_sched_barrier(0);   // keeps the live operands few
     }
-    f16x8 mn[NM];
-    float d[NM], dm[NM];
+    f16x8 mn[kGuBlocks];
+    float d[kGuBlocks], dm[kGuBlocks];
 #pragma unroll
-    for (int g = 0; g < NM; g++) {
+    for (int g = 0; g < kGuBlocks; g++) {
         const uint4 hw = *(const uint4 *)(rw + g * gstride);
         mn[g] = q4_mins_f16(hw);
         d[g] = h2f(hw.x) * 16384.f;              // codes entered times 2^-14
@@ -1152,7 +1152,7 @@ FO_DEV void q4_super_block(f32x4 (&acc)[NM][NB], const uint8_t *rw, uint32_t gst
         // A: the sums of token 16 tb + col: hi, mid, lo terms of the eight sub-blocks, zeros
         const f16x8 sa = *(const f16x8 *)(sb + (16 * tb + col) * 64 + 16 * kg);
 #pragma unroll
-        for (int g = 0; g < NM; g++) {
+        for (int g = 0; g < kGuBlocks; g++) {
             const f32x4 ms = __builtin_amdgcn_mfma_f32_16x16x32_f16(sa, mn[g], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[g][tb][i] = fmaf(d[g], dd[g][tb][i], fmaf(dm[g], ms[i], acc[g][tb][i]));
@@ -1239,9 +1239,9 @@ __global__ __launch_bounds__(64 * kGuWaves, 2) void k_pf_gateup_f16(PrefillArgs 
         };
         auto run = [&](auto NBC) {
             constexpr int NB = decltype(NBC)::value;
-                        f32x4 acc[4][NB];                                  // gate rows 0..15, 16..31, up rows 0..15, 16..31
+            f32x4 acc[kGuBlocks][NB];                          // gate rows 0..15, 16..31, up rows 0..15, 16..31
 #pragma unroll
-            for (int g = 0; g < 4; g++)
+            for (int g = 0; g < kGuBlocks; g++)
 #pragma unroll
                 for (int tb = 0; tb < NB; tb++) acc[g][tb] = (f32x4){0.f, 0.f, 0.f, 0.f};
             for (int q = 0; q < NQ; q++) {
@@ -1249,7 +1249,7 @@ __global__ __launch_bounds__(64 * kGuWaves, 2) void k_pf_gateup_f16(PrefillArgs 
                 issue_x(q);
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();                               // everyone's loads of step q have landed
-                q4_super_block<4, NB>(acc, wb + col * 144, kGuHalf, gu_lds, aoff, sb, col, kg);
+                q4_super_block<NB>(acc, wb + col * 144, kGuHalf, gu_lds, aoff, sb, col, kg);
                 __syncthreads();                               // the step's LDS is free for the next one
             }
 #pragma unroll
@@ -1638,8 +1638,7 @@ __global__ __launch_bounds__(kPfD16Waves * 64, kPfD16PerCU * kPfD16Waves / 4) vo
 #pragma clang fp contract(on)
 
 // ------------------------------------------------------------ Q6_K down of the thin tiles
-// Tiles of at most kPfThin pairs (k_pf_group orders them last) run the
-// decode matvec's integer path instead of k_pf_down16: a 16-row weight tile
+// Tiles of at most kPfThin thin pairs (k_pf_group's ttiles) run the decode matvec's integer path instead of k_pf_down16: a 16-row weight tile
 // streamed with 1 KiB loads into LDS (the next tile in flight) and, per pair,
 // the Q6_K super-block dot on v_mfma_i32_16x16x64_i8 against the pair's
 // activation as int8 limbs (q6k_mfma.h, as k_matvec_q6k_tile). The limbs are
@@ -1648,12 +1647,13 @@ __global__ __launch_bounds__(kPfD16Waves * 64, kPfD16PerCU * kPfD16Waves / 4) vo
 // applied to the result. The code building is shared by the tile's pairs, so
 // a weight costs ~0.75 + 0.5 n VALU instructions per code against ~3.4 for
 // the fp16 operand decode of k_pf_down16, whose 16-token MFMA blocks a thin
-// tile leaves mostly empty. Work unit = (thin tile, kPfThinWaves *
-// kPfThinTPW * 16 rows): the work-group's waves prepare one pair's
-// activation each into LDS shared by all of them (one copy per work-group,
-// so that 8 waves per CU fit in LDS: with a copy per one-wave work-group
-// only 5 did: 121.5 -> 109.3 us at config 5), then each wave streams its
-// kPfThinTPW tiles; units dealt round-robin; F == 1024. (4 waves x 4 tiles,
+// tile leaves mostly empty. Work unit = (thin tile, 512 rows, or 256 or 128 where
+// few thin tiles leave work-groups without one): the work-group's waves prepare
+// one pair's activation each into LDS shared by all of them (one copy per
+// work-group, so that 8 waves per CU fit in LDS: with a copy per one-wave
+// work-group only 5 did: 121.5 -> 109.3 us for 512 tokens of 512 experts), then
+// each wave streams its tiles, kPfThinTPW or fewer; units dealt round-robin;
+// F == 1024. (4 waves x 4 tiles,
 // 8 x 4, 8 x 2, 2 x 8: 115 / 119 / 127 / 122 us; the results held in LDS
 // and stored once per unit: no change.)
 constexpr int kPfThinTPW = 8, kPfThinWaves = 4;
