@@ -738,7 +738,7 @@ static std::array<fo::PfBuf, 13> prefill_bufs(gpu_ctx_t *ctx, int T, int Tc, int
         buf(ctx->pf_tiles, ctx->pf_tiles_cap,
             sizeof(int32_t) * (8 * prefill_tile_cap(Tc, k, E, sh) + 4 * (size_t)fo::prefill_max_thin(Tc, k, E, sh))),
         buf(ctx->pf_ntiles, ctx->pf_ntiles_cap, 256),
-        buf(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)((Tc + chunk - 1) / chunk) * E),
+        buf(ctx->pf_segs, ctx->pf_segs_cap, sizeof(int32_t) * (size_t)fo::prefill_segments(Tc, chunk) * E),
         buf(ctx->pf_act, ctx->pf_act_cap, 2 * sizeof(uint16_t) * Pact),
         // the shared pass's output [Tc x H] (its down rows, pairs in token order)
         buf(ctx->pf_ys, ctx->pf_ys_cap, own ? sizeof(float) * (size_t)Tc * H : 0),

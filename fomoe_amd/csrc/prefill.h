@@ -14,6 +14,7 @@ namespace fo {
 
 constexpr int kPfMT = 64;        // tokens per GEMM tile (4 MFMA row blocks of 16)
 constexpr int kPfGroupLds = 16384;   // words of each grouping table (n_experts * ceil(tokens / 32))
+constexpr int kPfSeg = 512;          // tokens per grouping segment of a larger pass, at most
 constexpr int kPfMaxPairs = 1 << 17; // pairs of a pass (its down outputs: 2 GiB at n_embd 4096)
 constexpr int kPfThin = 4;       // pairs of a thin tile (integer-MFMA Q6_K down path)
 constexpr int kPfGateWaves = 8;                   // gate/up work-group: 4 gate + 4 up waves (two per CU)
@@ -48,8 +49,8 @@ struct PrefillArgs {
     int32_t *ttiles;             // [max_thin x 4] {expert, first pair, n} of up to kPfThin thin pairs
     int32_t *n_tiles;            // [6]: tiles, thin tiles, work counter of the gate/up kernel, double
                                  // tiles, unused, the shared expert's first tile
-    int32_t *segs;               // [ceil(T / chunk) x E] pairs per (chunk, expert), then their first pair
-                                 // slots (passes above the grouping table's size)
+    int32_t *segs;               // [prefill_segments(T, chunk) x E] pairs per (segment, expert), then their
+                                 // first pair slots (passes above the grouping table's size)
     int chunk;                   // tokens per chunk (prefill_chunk_tokens of the layer; a pass starts at one)
     int max_tiles;
     uint16_t *act_hi, *act_lo;   // [P x F] SwiGLU activation as bf16 hi + lo terms (a Q6_K
@@ -102,6 +103,11 @@ inline int prefill_most_tokens(int k, bool shared) { return kPfMaxPairs / (k + (
 inline int prefill_chunk_tokens(int k, int E, bool shared) {
     const int table = (kPfGroupLds / E) * 32, most = prefill_most_tokens(k, shared);
     return table < most ? table : most;
+}
+// Segments of a pass: each chunk in kPfSeg tokens and what is left of it.
+inline int prefill_segments(int T, int chunk) {
+    const int per = (chunk + kPfSeg - 1) / kPfSeg;
+    return T / chunk * per + (T % chunk + kPfSeg - 1) / kPfSeg;
 }
 inline int prefill_pass_tokens(int k, int E, bool shared) {
     const int c = prefill_chunk_tokens(k, E, shared);
